@@ -186,7 +186,10 @@ size_t teeny_flash_attn2_bwd_workspace_bytes(int n_ctx_q, int batch, int n_heads
  * sums a merge kernel adds in a fixed order; otherwise equal to the above.
  * With a smaller workspace such a backward runs its dK/dV in two wavefront
  * groups per workgroup instead (the form used from 2048 to 12287 query rows
- * of even groups).  No counterpart in the reference. */
+ * of even groups).  fp32: the workspace that lets up to 32 dK/dV workgroups
+ * share the walk of a 64-key block where that brings the grid to four
+ * workgroups per CU, merged the same way; with a smaller one a single
+ * workgroup walks it.  No counterpart in the reference. */
 size_t teeny_flash_attn2_bwd_workspace_bytes_gqa(int n_ctx_q, int n_ctx_k, int batch,
                                                  int n_heads_q, int n_heads_kv, int head_dim,
                                                  int dtype);

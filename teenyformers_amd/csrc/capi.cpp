@@ -303,9 +303,12 @@ int fa2_fwd(bool causal, const void* q, const void* k, const void* v, void* o, f
     return launch(name, dim3(tot), dim3(threads), 0, stream, args);
   }
   if (o_merged || rope_cs) return TEENY_ERR_UNSUPPORTED;
+  int heads = batch * hq;
+  long wgs = (long)((n_ctx_q + 63) / 64) * heads;
+  if (wgs >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   snprintf(name, sizeof name, "teeny_fa2_fwd_f32_d%d_%s", head_dim, cz);
-  void* args[] = {&q, &k, &v, &o, &l, &n_ctx_q, &n_ctx_k, &scale, &hq, &hkv};
-  return launch(name, dim3((n_ctx_q + 63) / 64, batch * hq), dim3(64), 0, stream, args);
+  void* args[] = {&q, &k, &v, &o, &l, &n_ctx_q, &n_ctx_k, &scale, &hq, &hkv, &heads};
+  return launch(name, dim3((unsigned)wgs), dim3(256), 0, stream, args);
 }
 
 // bf16: per (b, q head) and block of 32 query rows, 32 values of -LSE/scale
@@ -374,6 +377,19 @@ size_t dkdv_split_bytes(int n_ctx_k, int batch, int hkv, int head_dim, int split
   return align256(2 * (size_t)split * batch * hkv * n_ctx_k * head_dim * sizeof(float));
 }
 
+// fp32 dK/dV: how many workgroups share the walk of a 64-key block over its
+// group's 32-row q tiles: as many as bring the grid to four workgroups per CU
+// (measured, forward + backward: B1 Hq8 Hkv1 Sq396 Sk59 D128 65 us against
+// ~110 unshared; B1 Hq32 Hkv8 S706 D32 115, 123 at two per CU and 155 at
+// one), at most 32 and at least four tiles each; the merge reads every share.
+int dkdv_f32_split(int n_ctx_q, int n_ctx_k, int batch, int hq, int hkv) {
+  const long wgs = (long)((n_ctx_k + 63) / 64) * batch * hkv;
+  const long items = (long)(hq / hkv) * ((n_ctx_q + 31) / 32);
+  const long want = 4L * device_cus() / wgs, most = items / 4;
+  const long s = want < most ? want : most;
+  return s < 1 ? 1 : s > 32 ? 32 : (int)s;
+}
+
 int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void* o,
             const void* dout, const float* l, void* dq, void* dk, void* dv, int n_ctx_q,
             int n_ctx_k, float scale, int batch, int hq, int hkv, int head_dim, int dtype,
@@ -389,7 +405,6 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
   if (!scale_ok(scale, dtype)) return TEENY_ERR_INVALID_VALUE;
   if (!workspace || workspace_bytes < fa2_bwd_ws(n_ctx_q, batch, hq, head_dim, dtype))
     return TEENY_ERR_WORKSPACE;
-  const long rows = (long)batch * hq * n_ctx_q;
   float* delta = (float*)workspace;
   const char* cz = causal ? "c" : "n";
   char name[64];
@@ -442,18 +457,33 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
     return launch(*gsfx ? "teeny_fa2_dkdv_merge_bf16_g32" : "teeny_fa2_dkdv_merge_bf16", dim3((unsigned)((n / 8 + 255) / 256)), dim3(256),
                   0, stream, a3);
   }
-  snprintf(name, sizeof name, "teeny_fa2_bwd_pre_f32_d%d", head_dim);
-  void* a0[] = {&o, &dout, &delta, (void*)&rows};
-  rc = launch(name, dim3((unsigned)((rows + 255) / 256)), dim3(256), 0, stream, a0);
-  if (rc) return rc;
+  // dQ first: it also writes Delta = rowsum(O * dO) for the dK/dV kernel
+  int heads = batch * hq, kv_heads = batch * hkv;
+  void* a1[] = {&q,     &k,  &v,       &o,       &dout,  &l,
+                &delta, &dq, &n_ctx_q, &n_ctx_k, &scale, &hq, &hkv, &heads};
+  const long wgs_q = (long)((n_ctx_q + 63) / 64) * heads;
+  const long wgs_k = (long)((n_ctx_k + 63) / 64) * kv_heads;
+  if (wgs_q >= (1L << 31) || wgs_k * 32 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   snprintf(name, sizeof name, "teeny_fa2_bwd_dq_f32_d%d_%s", head_dim, cz);
-  void* a1[] = {&q, &k, &v, &dout, &l, &delta, &dq, &n_ctx_q, &n_ctx_k, &scale, &hq, &hkv};
-  rc = launch(name, dim3((n_ctx_q + 63) / 64, batch * hq), dim3(64), 0, stream, a1);
+  rc = launch(name, dim3((unsigned)wgs_q), dim3(256), 0, stream, a1);
   if (rc) return rc;
+  // dK, dV: the walk over the group's q tiles shared out where the workspace
+  // holds the partial sums (and the merge may store whole vectors)
+  const size_t base = fa2_bwd_ws(n_ctx_q, batch, hq, head_dim, dtype);
+  int share = dkdv_f32_split(n_ctx_q, n_ctx_k, batch, hq, hkv);
+  if ((((uintptr_t)dk | (uintptr_t)dv | (uintptr_t)workspace) & 15) != 0 ||
+      workspace_bytes < base + dkdv_split_bytes(n_ctx_k, batch, hkv, head_dim, share))
+    share = 1;
+  float* part = share > 1 ? (float*)((char*)workspace + base) : nullptr;
   snprintf(name, sizeof name, "teeny_fa2_bwd_dkdv_f32_d%d_%s", head_dim, cz);
-  void* a2[] = {&q,  &k,  &v,       &dout,    &l,     &delta, &dk,
-                &dv, &n_ctx_q, &n_ctx_k, &scale, &hq,    &hkv};
-  return launch(name, dim3((n_ctx_k + 63) / 64, batch * hkv), dim3(64), 0, stream, a2);
+  void* a2[] = {&q,  &k,    &v,       &dout,    &l,     &delta, &dk,
+                &dv, &part, &n_ctx_q, &n_ctx_k, &scale, &hq,    &hkv, &kv_heads, &share};
+  rc = launch(name, dim3((unsigned)(wgs_k * share)), dim3(256), 0, stream, a2);
+  if (rc || share == 1) return rc;
+  long n = (long)batch * hkv * n_ctx_k * head_dim;  // a multiple of 8
+  void* a3[] = {&part, &dk, &dv, &n, &share, &scale};
+  return launch("teeny_fa2_dkdv_merge_bf16_g32", dim3((unsigned)((n / 8 + 255) / 256)), dim3(256),
+                0, stream, a3);
 }
 
 // ---------------------------------------------------------------------------
@@ -649,9 +679,11 @@ size_t teeny_flash_attn2_bwd_workspace_bytes_gqa(int n_ctx_q, int n_ctx_k, int b
       head_dim <= 0 || n_heads_q % n_heads_kv != 0)
     return 0;
   dtype &= ~TEENY_GRAD_F32;
-  // the split is planned only for the causal backward
+  // the bf16 split is planned only for the causal backward
   const int split =
-      dkdv_plan(true, n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv, dtype).split;
+      dtype == TEENY_F32
+          ? dkdv_f32_split(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv)
+          : dkdv_plan(true, n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv, dtype).split;
   return fa2_bwd_ws(n_ctx_q, batch, n_heads_q, head_dim, dtype) +
          dkdv_split_bytes(n_ctx_k, batch, n_heads_kv, head_dim, split);
 }

@@ -141,6 +141,48 @@ def test_fa2_f32_fwd_bwd(cuda, shape, causal):
         assert err <= F32_TOL, f"{name} {err}"
 
 
+F32_EDGES = [  # B, Hq, Hkv, Sq, Sk, D: 16-row wavefronts, 32-row tiles, 64-row workgroups
+    (1, 1, 1, 1, 1, 64),
+    (2, 2, 2, 15, 17, 128),
+    (1, 2, 1, 16, 31, 32),
+    (1, 2, 2, 33, 32, 16),
+    (1, 4, 2, 63, 65, 64),
+    (1, 1, 1, 97, 128, 8),
+    (1, 8, 1, 200, 70, 64),     # the dK/dV walk shared out over workgroups
+    (2, 4, 1, 161, 161, 128),   # ... unevenly
+]
+
+
+@pytest.mark.parametrize("shape", F32_EDGES)
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("aligned", [True, False])
+def test_fa2_f32_edges(cuda, shape, causal, aligned):
+    """Tile and wavefront edges against the oracle; tensors that start 4 bytes
+    past a 16-byte boundary take the kernels' register copy.  The gradients
+    sum up to group * Sq fp32 terms: the flat bar scaled by the largest one."""
+    B, Hq, Hkv, Sq, Sk, D = shape
+
+    def put(a):
+        t = torch.empty(a.size + 1, dtype=torch.float32, device="cuda")[0 if aligned else 1:]
+        t = t[:a.size].view(a.shape)
+        t.copy_(torch.from_numpy(a))
+        return t
+
+    q, k, v, do = inputs(30, *shape, bf16=False)
+    scale = 1.0 / math.sqrt(D)
+    qd, kd, vd, dod = (put(t) for t in (q, k, v, do))
+    o, lse = ops.flash_attn2_fwd(qd, kd, vd, scale, causal, out=put(np.zeros_like(q)))
+    oe, le = O.fa2_fwd(q, k, v, scale, causal)
+    assert np.abs(host(o) - oe).max() <= F32_TOL
+    assert np.abs(host(lse) - le).max() <= F32_TOL
+    grads = ops.flash_attn2_bwd(qd, kd, vd, put(oe), lse, dod, scale, causal,
+                                dq=put(np.zeros_like(q)), dk=put(np.zeros_like(k)),
+                                dv=put(np.zeros_like(v)))
+    for name, got, want in zip(("dq", "dk", "dv"), grads, O.fa2_bwd(q, k, v, oe, do, le, scale, causal)):
+        err = float(np.abs(host(got) - want).max())
+        assert err <= F32_TOL * max(1.0, float(np.abs(want).max())), f"{name} {err}"
+
+
 # ---------------------------------------------------------------------------
 # bf16 MFMA path
 # ---------------------------------------------------------------------------
