@@ -395,8 +395,9 @@ int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F
  * a multiple of 4; x and w 16-byte aligned. */
 int teeny_linear_f32(const void* x, const void* w, void* y, int M, int N, int K,
                      hipStream_t stream);
-/* This library's fp32 GEMM for the same product: each output one fp32
- * fused multiply-add chain over k in increasing order. */
+/* This library's fp32 GEMM for the same product: each output fp32 fused
+ * multiply-adds over k, in one chain of increasing k above 64 rows, in eight
+ * chains added in order up to 64 rows (the same for any M there). */
 int teeny_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K,
                    hipStream_t stream);
 

@@ -2,19 +2,22 @@
 // precision (teeny-core's Linear behind sym_linear, src/layers/mod.rs:54-58,
 // runs in fp32; src/loader.rs:41,66-80 decodes every weight to f32).
 //
-// teeny_linear_f32 hands its products to hipBLASLt; this kernel is the
+// teeny_linear_f32 hands its products to hipBLASLt; these kernels are the
 // library's own path where hipBLASLt does not take the device, shape or
-// stream (a product under graph capture).  Each output is one fp32 fused
+// stream (a product under graph capture).
+//
+// Up to 64 rows (a decode step, one row per sequence): teeny_gemm_f32_sk_*,
+// below.  More rows: teeny_gemm_f32_nt, each output one fp32 fused
 // multiply-add chain over k in increasing order, so the result does not
 // depend on the tiling.
 //
-// Tiling: a workgroup of 256 threads owns a 128 x 128 tile of y; 16-deep K
+// Tiling of teeny_gemm_f32_nt: a workgroup of 256 threads owns a 128 x 128 tile of y; 16-deep K
 // slices of x and w are staged in LDS transposed (k-major), two buffers, so
 // the next slice's global loads are in flight while the current one is
 // multiplied; each thread accumulates an 8 x 8 block (rows ty*4 + {0..3} and
 // 64 + ty*4 + {0..3}, columns likewise from tx) with 16-byte LDS reads.
 // Rows past M or N and k past K load zeros and are never stored.
-#include "common.h"
+#include "cdna4.h"
 
 namespace {
 
@@ -110,3 +113,153 @@ extern "C" __global__ __launch_bounds__(256) void teeny_gemm_f32_nt(
     }
   }
 }
+
+// ---------------------------------------------------------------------------
+// Few rows: y[M, N] = x[M, K] . w[N, K]^T, M <= 16 MT, bound by reading w once.
+//
+// A workgroup of 8 wavefronts owns 16 RT rows of w; the wavefronts take its
+// 64-wide k chunks in turn (8 c + wavefront), so that each CU streams whole
+// rows and the loop has no barrier, and their sums are added in wavefront
+// order through LDS.  w rows are the A operand of v_mfma_f32_16x16x4_f32 and x
+// rows the B operand: a 16-byte load of a lane (row l % 16, k = 4 (l / 16)) of
+// each feeds four products (the k order inside 16 only has to agree).  The k
+// order does not depend on RT and MT, so neither do the bits of an output on M.
+// Rows past M or N repeat the last one and are not stored; the k past K of the
+// last chunk load zeros.
+//
+// Measured from HBM (weights rotated past the last-level cache), 16 wavefronts
+// per CU at M = 1: N32000 K2048 46 us (5.7 TB/s), N28672 K4096 83 us (5.7),
+// N4096 K14336 41 us (5.7), N2048 K8192 21 us, N3072 K2048 8 us; the 128 x 128
+// tiles took 0.5 ms each (2 ms at K8192).  Two or more chunks per register
+// set, or two row tiles, leave one workgroup per CU and lost 2-20 % there; at
+// M = 16 the x loads cost as much as w's, and two row tiles (half the x loads)
+// gain up to 12 % once the grid still fills the CUs twice, and up to 25 % at
+// M = 64.
+// ---------------------------------------------------------------------------
+namespace {
+
+DEVI f32x4 mfma4(float a, float b, f32x4 c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
+}
+
+constexpr int SKW = 8;   // wavefronts per workgroup
+constexpr int SKC = 64;  // k per chunk
+
+template <int RT, int MT>
+__device__ __forceinline__ void gemm_f32_sk(const float* __restrict__ x,
+                                            const float* __restrict__ w, float* __restrict__ y,
+                                            int M, int N, int K) {
+  __shared__ __attribute__((aligned(16))) float red[SKW][RT * MT][64][4];
+  const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long row0 = (long)blockIdx.x * (16 * RT);
+  const float* wr[RT];
+  const float* xr[MT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r) wr[r] = w + min(row0 + 16 * r + j, (long)N - 1) * K + 4 * g;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) xr[m] = x + (long)min(16 * m + j, M - 1) * K + 4 * g;
+  f32x4 acc[RT][MT];
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) acc[r][m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 a[2][4][RT], b[2][4][MT];  // two register sets of a chunk
+  auto load = [&](int set, int c) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = c * SKC + 16 * u;
+#pragma unroll
+      for (int r = 0; r < RT; ++r) a[set][u][r] = *reinterpret_cast<const f32x4*>(wr[r] + k);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) b[set][u][m] = *reinterpret_cast<const f32x4*>(xr[m] + k);
+    }
+    // every load is issued before the products that follow wait for one
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto products = [&](int set) __attribute__((always_inline)) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int r = 0; r < RT; ++r)
+#pragma unroll
+          for (int m = 0; m < MT; ++m)
+            acc[r][m] = mfma4(a[set][u][r][e], b[set][u][m][e], acc[r][m]);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // this wavefront's whole chunks, the next one's loads in flight
+  // (straight-line bodies: a branch around the loads would make the products
+  // wait for all of them)
+  const int n = max(0, (K / SKC - wave + SKW - 1) / SKW);
+  int c = wave;
+  if (n > 0) {
+    int i = 0;
+    load(0, c);
+    for (; i + 2 < n; i += 2, c += 2 * SKW) {
+      load(1, c + SKW);
+      products(0);
+      load(0, c + 2 * SKW);
+      products(1);
+    }
+    if (i + 1 < n) {
+      load(1, c + SKW);
+      products(0);
+      products(1);
+      c += 2 * SKW;
+    } else {
+      products(0);
+      c += SKW;
+    }
+  }
+  // the last chunk of K, if it is not whole; K is a multiple of 4, so a load
+  // is within K or past it
+  if (c * SKC < K) {
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      const int k = c * SKC + 16 * u;
+      const bool in = k + 4 * g < K;
+#pragma unroll
+      for (int r = 0; r < RT; ++r)
+        a[0][u][r] = in ? *reinterpret_cast<const f32x4*>(wr[r] + k) : f32x4{0, 0, 0, 0};
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+        b[0][u][m] = in ? *reinterpret_cast<const f32x4*>(xr[m] + k) : f32x4{0, 0, 0, 0};
+    }
+    products(0);
+  }
+#pragma unroll
+  for (int r = 0; r < RT; ++r)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) *reinterpret_cast<f32x4*>(red[wave][r * MT + m][lane]) = acc[r][m];
+  __syncthreads();
+  // output (row 16 r + 4 g + i of w, row 16 m + j of x) is value i of lane
+  // (j, g) of block (r, m): one lane of the workgroup per four w rows
+  for (int t = threadIdx.x; t < RT * MT * 64; t += 64 * SKW) {
+    const int blk = t >> 6, l = t & 63;
+    f32x4 s = *reinterpret_cast<const f32x4*>(red[0][blk][l]);
+#pragma unroll
+    for (int v = 1; v < SKW; ++v) s += *reinterpret_cast<const f32x4*>(red[v][blk][l]);
+    const int m = 16 * (blk % MT) + (l & 15);
+    const long n = row0 + 16 * (blk / MT) + 4 * (l >> 4);
+    if (m >= M) continue;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (n + i < N) y[(long)m * N + n + i] = s[i];
+  }
+}
+
+}  // namespace
+
+#define TEENY_GEMM_F32_SK(RT, MT)                                                          \
+  extern "C" __global__ __launch_bounds__(64 * SKW) void teeny_gemm_f32_sk_r##RT##_m##MT( \
+      const float* x, const float* w, float* y, int M, int N, int K) {                     \
+    gemm_f32_sk<RT, MT>(x, w, y, M, N, K);                                                 \
+  }
+TEENY_GEMM_F32_SK(1, 1)
+TEENY_GEMM_F32_SK(2, 1)
+TEENY_GEMM_F32_SK(1, 2)
+TEENY_GEMM_F32_SK(2, 2)
+TEENY_GEMM_F32_SK(1, 4)
+TEENY_GEMM_F32_SK(2, 4)

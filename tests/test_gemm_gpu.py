@@ -194,6 +194,21 @@ def test_linear_f32_llama_shapes(cuda, M, N, K, entry):
     print(f"linear_f32 {entry} M{M} N{N} K{K}: rel-L2 {rel:.2e}", flush=True)
 
 
+@pytest.mark.parametrize("M", [1, 9, 16, 17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(1, 4), (15, 60), (17, 64), (16390, 68), (48, 512), (33, 1028)])
+def test_gemm_f32_few_rows(cuda, M, N, K):
+    """The few-row kernel at the edges of its row tiles, of N (single and
+    paired row tiles) and of the K chunks shared out over 8 wavefronts; an
+    output's bits do not depend on M."""
+    x, w = _operands_f32(64, N, K, seed=M + N + K)
+    xd, wd = torch.from_numpy(x).cuda(), torch.from_numpy(w).cuda()
+    y = _gemm_f32(xd[:M], wd, "teeny_gemm_f32")
+    x64, w64 = x[:M].astype(np.float64), w.astype(np.float64)
+    bound = 2.0 * K * 2.0 ** -24 * (np.abs(x64) @ np.abs(w64).T)
+    assert np.all(np.abs(y.cpu().numpy() - x64 @ w64.T) <= bound)
+    assert torch.equal(y, _gemm_f32(xd, wd, "teeny_gemm_f32")[:M])
+
+
 def test_linear_f32_op(cuda):
     """ops.linear routes fp32 products (no gradient) through teeny_linear_f32,
     not torch; ops.gemm_f32 is the own kernel."""
