@@ -1011,9 +1011,7 @@ int teeny_decode_qkv_attention_dev(const float* parts, int n_parts, void* k_cach
   return launch(name, dim3((unsigned)(batch * n_heads_kv)), dim3(512), 0, stream, args);
 }
 
-static int decode_chunks(int n_keys) { return (n_keys + 255) / 256; }  // fp32 kernel
-
-// bf16 matrix-core kernel: keys per wavefront chosen so that one step runs
+// matrix-core kernels: keys per wavefront chosen so that one step runs
 // about 1024 wavefronts (a multiple of the 32-key tile, 64 .. 1024).  At the
 // Llama-8B decode shape (B16, 8 kv heads, 640 cached rows) that is 96 keys
 // per wavefront: attention + combine 11.3-12.1 us per layer, against
@@ -1056,10 +1054,10 @@ static int decode_attention_impl(const void* q, const void* k_cache, const void*
     return TEENY_ERR_WORKSPACE;
   // the matrix-core kernel addresses one (b, kv head) cache slab with 32-bit
   // byte offsets
-  const bool mfma = dtype == TEENY_BF16 && (head_dim == 64 || head_dim == 128) &&
-                    (long)cache_len * head_dim * 2 < (1L << 31);
+  const bool mfma = dtype == TEENY_F32 || ((head_dim == 64 || head_dim == 128) &&
+                                           (long)cache_len * head_dim * 2 < (1L << 31));
   const int per = mfma ? decode_keys_per_split(n_keys, batch, n_heads_kv) : 256;
-  int n_chunks = mfma ? (n_keys + per - 1) / per : decode_chunks(n_keys);
+  int n_chunks = (n_keys + per - 1) / per;
   size_t rows = (size_t)batch * n_heads_q * n_chunks;
   float* pm = (float*)workspace;
   float* pl = (float*)((char*)workspace + align256(rows * sizeof(float)));
@@ -1067,16 +1065,16 @@ static int decode_attention_impl(const void* q, const void* k_cache, const void*
   char name[48];
   int rc;
   if (mfma) {
-    snprintf(name, sizeof name, "teeny_decode_mfma_bf16_d%d", head_dim);
+    snprintf(name, sizeof name,
+             dtype == TEENY_F32 ? "teeny_decode_f32_d%d" : "teeny_decode_mfma_bf16_d%d", head_dim);
     int per_split = per;
     void* a0[] = {&q,  &k_cache, &v_cache, &pm,        &pl,        &po,           &n_heads_q,
                   &n_heads_kv, &n_past,  &n_keys,   &cache_len, &per_split, &softmax_scale};
     rc = launch(name, dim3(n_chunks, batch * n_heads_kv), dim3(64), 0, stream, a0);
   } else {
-    snprintf(name, sizeof name, "teeny_decode_attn_partial_%s", dtype_tag(dtype));
     void* a0[] = {&q,      &k_cache, &v_cache,   &pm,       &pl,           &po, &n_heads_q,
                   &n_heads_kv, &n_past, &n_keys, &cache_len, &head_dim, &softmax_scale};
-    rc = launch(name, dim3(n_chunks, batch * n_heads_kv), dim3(256), 0, stream, a0);
+    rc = launch("teeny_decode_attn_partial_bf16", dim3(n_chunks, batch * n_heads_kv), dim3(256), 0, stream, a0);
   }
   if (rc) return rc;
   snprintf(name, sizeof name, "teeny_decode_attn_combine_%s", dtype_tag(dtype));

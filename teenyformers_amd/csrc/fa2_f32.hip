@@ -42,32 +42,13 @@
 // Tiles of 32 rows stream into LDS by buffer_load ... lds one tile ahead (two
 // buffers); the 16-byte chunks of a row are XOR-permuted so that 16 rows read
 // at one chunk, and 16 chunks of one row, fall into distinct banks.
-#include "cdna4.h"
+#include "f32_mfma.h"
 
 namespace {
 
 constexpr int kWaves = 4;            // wavefronts per workgroup
 constexpr int kRows = 16 * kWaves;   // query (or key) rows per workgroup
 constexpr int kTile = 32;            // rows per LDS tile
-
-DEVI f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
-// the value held by lane l ^ 16
-DEVI float other_16(float x) {
-  auto r = __builtin_amdgcn_permlane16_swap(__builtin_bit_cast(unsigned, x),
-                                            __builtin_bit_cast(unsigned, x), false, false);
-  return __builtin_bit_cast(float, (threadIdx.x & 16) ? r[0] : r[1]);
-}
-// over the four lanes that share j
-DEVI float max_g(float x) {
-  x = fmaxf(x, other_16(x));
-  return fmaxf(x, other_half(x));
-}
-DEVI float sum_g(float x) {
-  x += other_16(x);
-  return x + other_half(x);
-}
 
 // 16-byte chunk index of chunk c of tile row r: rows of D / 4 chunks, the
 // chunk XORed with the row's line (256 bytes) so that 16 consecutive rows'
@@ -81,18 +62,11 @@ DEVI int chunk_at(int r, int c) {
 }
 
 template <int D>
-struct Geo {
-  static constexpr int CPR = D / 4;                  // 16-byte chunks per row
-  static constexpr int TILE = kTile * D * 4;         // bytes of a tile
-  static constexpr int NLD = TILE / 1024;            // 1 KiB loads per tile
-  static constexpr int NC = D < 16 ? 1 : D / 16;     // chunks of 16 d per row
-  static constexpr int VW = D >= 64 ? 4 : D == 32 ? 2 : 1;  // d per transposed read
-  static constexpr int NH = D < 16 ? 1 : D / (16 * VW);     // groups of VW output tiles
+struct Tile : Geo<D> {
+  static constexpr int CPR = D / 4;           // 16-byte chunks per row
+  static constexpr int TILE = kTile * D * 4;  // bytes of a tile
+  static constexpr int NLD = TILE / 1024;     // 1 KiB loads per tile
 };
-
-// global vectors: tensors may start at any float
-typedef float f32x4g __attribute__((ext_vector_type(4), aligned(4)));
-typedef float f32x2g __attribute__((ext_vector_type(2), aligned(4)));
 
 // Rows row0 .. row0 + 31 of a [n, D] head at `base` into LDS; rows at or past
 // n load as zeros (outside the descriptor's range).  The descriptor is built
@@ -111,16 +85,16 @@ DEVI void load_tile(const float* base, int row0, int n, char* lds, int wave, int
   }
   const auto rs = make_rsrc(base + (long)row0 * D, rows * D * 4);
 #pragma unroll
-  for (int i0 = 0; i0 < Geo<D>::NLD; i0 += kWaves) {
+  for (int i0 = 0; i0 < Tile<D>::NLD; i0 += kWaves) {
     const int i = i0 + wave;
-    if (i < Geo<D>::NLD) {
-      const int L = i * 64 + lane, r = L / Geo<D>::CPR, c = L % Geo<D>::CPR;
+    if (i < Tile<D>::NLD) {
+      const int L = i * 64 + lane, r = L / Tile<D>::CPR, c = L % Tile<D>::CPR;
       dma16(rs, lds + i * 1024, (uint32_t)chunk_at<D>(r, c) * 16, 0);
     }
   }
 }
 
-// A row-wise A or B operand of one row: chunk c's four d, from LDS ...
+// A row-wise A operand of one tile row: chunk c's four d
 template <int D>
 DEVI f32x4 row_chunk(const char* tile, int r, int c, int g) {
   if constexpr (D == 8) {
@@ -130,20 +104,6 @@ DEVI f32x4 row_chunk(const char* tile, int r, int c, int g) {
     return *reinterpret_cast<const f32x4*>(tile + chunk_at<D>(r, 4 * c + g) * 16);
   }
 }
-// ... and from global memory
-template <int D>
-DEVI void row_regs(const float* row, int g, f32x4* out) {
-#pragma unroll
-  for (int c = 0; c < Geo<D>::NC; ++c) {
-    if constexpr (D == 8) {
-      out[c] = g < 2 ? (f32x4)*reinterpret_cast<const f32x4g*>(row + 4 * g)
-                     : f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-    } else {
-      out[c] = *reinterpret_cast<const f32x4g*>(row + 16 * c + 4 * g);
-    }
-  }
-}
-
 // out[u] = (rows 16 u + i of the tile) . (the lane's column), u = 0, 1: two
 // independent chains
 template <int D>
@@ -218,39 +178,6 @@ DEVI void accumulate(const char* tile, const f32x4* p, int j, int g,
   __builtin_amdgcn_sched_barrier(0);
 }
 
-template <int D>
-DEVI void zero_acc(f32x4 (*acc)[Geo<D>::VW]) {
-#pragma unroll
-  for (int h = 0; h < Geo<D>::NH; ++h)
-#pragma unroll
-    for (int e = 0; e < Geo<D>::VW; ++e) acc[h][e] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
-}
-
-// the lane's column of acc, each value through f, to row [D]: output tile e
-// of group h holds d = 16 VW h + VW (4 g + r) + e
-template <int D, typename F>
-DEVI void store_col(float* row, const f32x4 (*acc)[Geo<D>::VW], int g, F&& f) {
-  constexpr int VW = Geo<D>::VW;
-#pragma unroll
-  for (int h = 0; h < Geo<D>::NH; ++h) {
-    if constexpr (VW == 1) {
-      if (D >= 16 || g < 2)
-        *reinterpret_cast<f32x4g*>(row + 4 * g) =
-            f32x4g{f(acc[0][0][0]), f(acc[0][0][1]), f(acc[0][0][2]), f(acc[0][0][3])};
-    } else {
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float* p = row + 16 * VW * h + VW * (4 * g + r);
-        if constexpr (VW == 4)
-          *reinterpret_cast<f32x4g*>(p) =
-              f32x4g{f(acc[h][0][r]), f(acc[h][1][r]), f(acc[h][2][r]), f(acc[h][3][r])};
-        else
-          *reinterpret_cast<f32x2g*>(p) = f32x2g{f(acc[h][0][r]), f(acc[h][1][r])};
-      }
-    }
-  }
-}
-
 // Work item of a workgroup: (rank, head), rank 0 a head's longest walk, all
 // heads' rank 0 first.  With a multiple of 8 heads one XCD (ids deal round
 // robin) sees whole heads.  Where everything is resident at once, the time is
@@ -281,8 +208,8 @@ __device__ __forceinline__ void fwd_f32(const float* __restrict__ q, const float
                                         float* __restrict__ lse, int nq, int nk, float scale,
                                         int hq, int hkv, int heads) {
   struct __attribute__((aligned(16))) Smem {
-    char k[2][Geo<D>::TILE];
-    char v[2][Geo<D>::TILE];
+    char k[2][Tile<D>::TILE];
+    char v[2][Tile<D>::TILE];
   };
   __shared__ Smem sm;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
@@ -369,8 +296,8 @@ __device__ __forceinline__ void bwd_dq_f32(const float* __restrict__ q,
                                            int nq, int nk, float scale, int hq, int hkv,
                                            int heads) {
   struct __attribute__((aligned(16))) Smem {
-    char k[2][Geo<D>::TILE];
-    char v[2][Geo<D>::TILE];
+    char k[2][Tile<D>::TILE];
+    char v[2][Tile<D>::TILE];
   };
   __shared__ Smem sm;
   const int lane = threadIdx.x & 63, j = lane & 15, g = lane >> 4;
@@ -454,8 +381,8 @@ __device__ __forceinline__ void bwd_dkdv_f32(const float* __restrict__ q,
                                              float scale, int hq, int hkv, int heads,
                                              int shares) {
   struct __attribute__((aligned(16))) Smem {
-    char q[2][Geo<D>::TILE];
-    char dout[2][Geo<D>::TILE];
+    char q[2][Tile<D>::TILE];
+    char dout[2][Tile<D>::TILE];
     float ld[2][2][kTile];  // LSE, Delta of the tile's rows
   };
   __shared__ Smem sm;

@@ -17,7 +17,7 @@
 // multiplied; each thread accumulates an 8 x 8 block (rows ty*4 + {0..3} and
 // 64 + ty*4 + {0..3}, columns likewise from tx) with 16-byte LDS reads.
 // Rows past M or N and k past K load zeros and are never stored.
-#include "cdna4.h"
+#include "f32_mfma.h"
 
 namespace {
 
@@ -137,10 +137,6 @@ extern "C" __global__ __launch_bounds__(256) void teeny_gemm_f32_nt(
 // M = 64.
 // ---------------------------------------------------------------------------
 namespace {
-
-DEVI f32x4 mfma4(float a, float b, f32x4 c) {
-  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-}
 
 constexpr int SKW = 8;   // wavefronts per workgroup
 constexpr int SKC = 64;  // k per chunk

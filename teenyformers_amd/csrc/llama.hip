@@ -13,12 +13,12 @@
 //   rows are written (the bf16 prompt attention then reads Q from qkv and
 //   rotates it as it loads it, with teeny_rope_table's (cos, sin)).
 //
-// teeny_decode_attn_*: one new query row per (b, q head) against the first
-//   n_keys cached keys (flash-decoding: split-K partials over 256-key chunks,
+// teeny_decode_attn_*, teeny_decode_f32_*: one new query row per (b, q head) against the first
+//   n_keys cached keys (flash-decoding: split-K partials over the keys,
 //   then a log-sum-exp merge).  The reference has no KV cache and recomputes
 //   the whole prefix every step (examples/llama_generate.rs:373-381); this is
 //   the same attention row evaluated once.
-#include "common.h"
+#include "f32_mfma.h"
 
 namespace {
 
@@ -314,6 +314,110 @@ __device__ void decode_partial(const T* __restrict__ q, const T* __restrict__ kc
   }
 }
 
+// fp32 on the fp32 matrix cores: one wavefront per (key split, b, kv head).
+// The q heads of the group (at most 16) are the columns of S^T = K Q^T; K and
+// V rows are read straight from the cache in operand order (16 rows x 64
+// bytes, and 4 whole rows, per load), 32 keys at a time with every load of
+// the tile in flight, so no LDS and no barrier.  Bound by reading the cache,
+// and at one sequence by the loads' latency, so the splits are as fine as the
+// workspace allows (64 keys) until about 1024 wavefronts run.
+// One sequence, 8 kv heads of 64, 521 keys: 6.2 us against 50.6 (one thread per
+// key, three workgroups per kv head); 8 sequences of 4001 keys: 33 us, 4.0 TB/s.
+template <int D>
+__device__ __forceinline__ void decode_f32(const float* __restrict__ q,
+                                           const float* __restrict__ kc,
+                                           const float* __restrict__ vc, float* __restrict__ pm,
+                                           float* __restrict__ pl, float* __restrict__ po, int hq,
+                                           int hkv, const int* __restrict__ n_past, int n_keys,
+                                           int cache_len, int keys_per_split, float scale) {
+  constexpr int NC = Geo<D>::NC, VW = Geo<D>::VW, NH = Geo<D>::NH;
+  const int lane = threadIdx.x, j = lane & 15, g = lane >> 4;
+  const int split = blockIdx.x, n_split = gridDim.x;
+  const int kvh = blockIdx.y, b = kvh / hkv, hk = kvh - b * hkv;
+  const int group = hq / hkv;
+  if (n_past) n_keys = min(min(*n_past + 1, n_keys), cache_len);
+  const int k0 = split * keys_per_split, k1 = min(k0 + keys_per_split, n_keys);
+  const long qh0 = (long)b * hq + (long)hk * group;  // first q head of the group
+  const float* kb = kc + (long)kvh * cache_len * D;
+  const float* vb = vc + (long)kvh * cache_len * D;
+  f32x4 qf[NC];
+  row_regs<D>(q + (qh0 + min(j, group - 1)) * D, g, qf);
+  f32x4 acc[NH][VW];
+  zero_acc<D>(acc);
+  float m = -INFINITY, l = 0.0f;
+  for (int t0 = k0; t0 < k1; t0 += 32) {
+    // rows at or past k1 re-read row k1 - 1; their P is zero
+    f32x4 kf[2][NC];
+    float vf[8][NH][VW];
+#pragma unroll
+    for (int u = 0; u < 2; ++u) row_regs<D>(kb + (long)min(t0 + 16 * u + j, k1 - 1) * D, g, kf[u]);
+#pragma unroll
+    for (int s = 0; s < 8; ++s) {
+      const float* row = vb + (long)min(t0 + 16 * (s >> 2) + 4 * g + (s & 3), k1 - 1) * D;
+#pragma unroll
+      for (int h = 0; h < NH; ++h) {
+        if constexpr (VW == 4) {
+          const f32x4 x = *reinterpret_cast<const f32x4g*>(row + 64 * h + 4 * j);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) vf[s][h][e] = x[e];
+        } else if constexpr (VW == 2) {
+          const f32x2 x = *reinterpret_cast<const f32x2g*>(row + 2 * j);
+          vf[s][h][0] = x[0];
+          vf[s][h][1] = x[1];
+        } else {
+          vf[s][h][0] = D == 8 && j >= 8 ? 0.0f : row[j];
+        }
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // every load is issued first
+    f32x4 s[2] = {};
+#pragma unroll
+    for (int c = 0; c < NC; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) s[u] = mfma4(kf[u][c][e], qf[c][e], s[u]);
+    float mx = -INFINITY;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[u][r] = t0 + 16 * u + 4 * g + r < k1 ? s[u][r] * scale : -INFINITY;
+        mx = fmaxf(mx, s[u][r]);
+      }
+    const float m_new = fmaxf(m, max_g(mx));  // the tile has a key below k1
+    const float alpha = expf(m - m_new);
+    m = m_new;
+    l *= alpha;
+#pragma unroll
+    for (int u = 0; u < 2; ++u)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        s[u][r] = expf(s[u][r] - m_new);
+        l += s[u][r];
+      }
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+      for (int e = 0; e < VW; ++e) acc[h][e] *= alpha;
+#pragma unroll
+    for (int x = 0; x < 8; ++x)
+#pragma unroll
+      for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int e = 0; e < VW; ++e)
+          acc[h][e] = mfma4(vf[x][h][e], s[x >> 2][x & 3], acc[h][e]);
+  }
+  l = sum_g(l);
+  if (j >= group) return;
+  const long row = (qh0 + j) * n_split + split;
+  if (g == 0) {
+    pm[row] = m;  // -inf for a split without keys
+    pl[row] = l;
+  }
+  store_col<D>(po + row * D, acc, g, [](float x) { return x; });
+}
+
 // grid B*Hq, block head_dim threads: merge the chunk partials.  The partials
 // of kGroup chunks are loaded together (one memory wait per group) and folded
 // into a running maximum: acc and l are scaled by e^(m_old - m_new) when a
@@ -489,12 +593,6 @@ TEENY_QKV_PARTS_INST(bf16, bf16)
     qkv_rope_rows<T>(qkv, q_out, k_cache, v_cache, seq, pos_dev, pos0, cache_len, hq, hkv,      \
                      head_dim, ln_base);                                                        \
   }                                                                                             \
-  extern "C" __global__ __launch_bounds__(256) void teeny_decode_attn_partial_##TN(            \
-      const T* q, const T* kc, const T* vc, float* pm, float* pl, float* po, int hq, int hkv,   \
-      const int* n_past, int n_keys, int cache_len, int head_dim, float scale) {                \
-    decode_partial<T>(q, kc, vc, pm, pl, po, hq, hkv, n_past, n_keys, cache_len, head_dim,      \
-                      scale);                                                                   \
-  }                                                                                             \
   extern "C" __global__ __launch_bounds__(256) void teeny_decode_attn_combine_##TN(            \
       const float* pm, const float* pl, const float* po, T* o, int n_chunks, int head_dim) {    \
     decode_combine<T>(pm, pl, po, o, n_chunks, head_dim);                                       \
@@ -503,6 +601,26 @@ TEENY_QKV_PARTS_INST(bf16, bf16)
       const T* x, long long* out, int cols) {                                                   \
     argmax_rows<T>(x, out, cols);                                                               \
   }
+
+// bf16 caches that the matrix-core kernel (decode_bf16.hip) does not take
+extern "C" __global__ __launch_bounds__(256) void teeny_decode_attn_partial_bf16(
+    const bf16* q, const bf16* kc, const bf16* vc, float* pm, float* pl, float* po, int hq,
+    int hkv, const int* n_past, int n_keys, int cache_len, int head_dim, float scale) {
+  decode_partial<bf16>(q, kc, vc, pm, pl, po, hq, hkv, n_past, n_keys, cache_len, head_dim, scale);
+}
+
+#define TEENY_DECODE_F32_INST(D)                                                                 \
+  extern "C" __global__ __launch_bounds__(64) void teeny_decode_f32_d##D(                       \
+      const float* q, const float* kc, const float* vc, float* pm, float* pl, float* po, int hq, \
+      int hkv, const int* n_past, int n_keys, int cache_len, int keys_per_split, float scale) {  \
+    decode_f32<D>(q, kc, vc, pm, pl, po, hq, hkv, n_past, n_keys, cache_len, keys_per_split,    \
+                  scale);                                                                       \
+  }
+TEENY_DECODE_F32_INST(8)
+TEENY_DECODE_F32_INST(16)
+TEENY_DECODE_F32_INST(32)
+TEENY_DECODE_F32_INST(64)
+TEENY_DECODE_F32_INST(128)
 
 TEENY_LLAMA_INST(f32, float)
 TEENY_LLAMA_INST(bf16, bf16)

@@ -255,6 +255,24 @@ def test_device_position_variants(cuda, dtype):
     assert torch.equal(kd, kc0) and torch.equal(vd, vc0)
 
 
+@pytest.mark.parametrize("B,Hq,Hkv,D,n_keys,L", [
+    (1, 1, 1, 64, 1, 4), (2, 4, 2, 64, 65, 65), (1, 16, 1, 128, 97, 120), (3, 6, 2, 32, 63, 64),
+    (1, 2, 2, 16, 130, 130), (2, 2, 1, 8, 33, 40), (1, 8, 2, 64, 4097, 4100)])
+def test_decode_attention_f32_edges(cuda, B, Hq, Hkv, D, n_keys, L):
+    """The fp32 decode kernel at the edges of its 16-key subtiles, 32-key tiles
+    and key splits, groups of 1 to 16 heads; rows past n_keys hold NaN.  Bar
+    of the fp32 attention: max abs 1e-5."""
+    g = torch.Generator(device="cuda").manual_seed(n_keys)
+    q = torch.randn(B, Hq, D, generator=g, device="cuda")
+    k, v = (torch.randn(B, Hkv, L, D, generator=g, device="cuda") for _ in range(2))
+    k[:, :, n_keys:] = v[:, :, n_keys:] = float("nan")
+    o = ops.decode_attention(q, k, v, n_keys)
+    kk, vv = (t[:, :, :n_keys].double().repeat_interleave(Hq // Hkv, 1) for t in (k, v))
+    p = ((kk @ q.double()[..., None])[..., 0] / D ** 0.5).softmax(-1)
+    want = (p[..., None] * vv).sum(2)
+    assert (o.double() - want).abs().max().item() <= 1e-5
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,L", [
     (4, 32, 8, 128, 640),   # the Llama-3-8B decode shape
     (3, 8, 1, 64, 300),     # 8 q heads on one kv head, cache off the 32-key tile
