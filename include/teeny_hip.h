@@ -186,13 +186,18 @@ size_t teeny_flash_attn2_bwd_workspace_bytes(int n_ctx_q, int batch, int n_heads
  * sums a merge kernel adds in a fixed order; otherwise equal to the above.
  * With a smaller workspace such a backward runs its dK/dV in two wavefront
  * groups per workgroup instead (the form used from 2048 to 12287 query rows
- * of even groups).  fp32: the workspace that lets up to 32 dK/dV workgroups
- * share the walk of a 64-key block where that brings the grid to four
- * workgroups per CU, merged the same way; with a smaller one a single
- * workgroup walks it.  No counterpart in the reference. */
+ * of even groups).  No counterpart in the reference. */
 size_t teeny_flash_attn2_bwd_workspace_bytes_gqa(int n_ctx_q, int n_ctx_k, int batch,
                                                  int n_heads_q, int n_heads_kv, int head_dim,
                                                  int dtype);
+/* The workspace that also lets several dK/dV workgroups share the walk of one
+ * key block over its query rows (fp32 partial sums, merged in a fixed order)
+ * where the key blocks alone would leave CUs idle; at least the above.  With a
+ * smaller workspace one workgroup walks each key block.  No counterpart in the
+ * reference. */
+size_t teeny_flash_attn2_bwd_workspace_bytes_shared(int n_ctx_q, int n_ctx_k, int batch,
+                                                    int n_heads_q, int n_heads_kv, int head_dim,
+                                                    int dtype);
 
 /* No counterpart in the reference: teeny_causal_flash_attn2_bwd for callers
  * that cannot allocate device memory (code under HIP graph capture, serving
@@ -390,8 +395,9 @@ int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F
 /* The same Linear in fp32, the reference's precision (teeny-core's Linear
  * behind sym_linear, src/layers/mod.rs:54-58, on the f32 weights that
  * src/loader.rs:41,66-80 decodes): hipBLASLt's fp32 GEMM (fp32 products
- * and accumulation, no workspace), or teeny_gemm_f32 where hipBLASLt does
- * not take the device or shape or the stream is capturing.  Any M and N; K
+ * and accumulation, no workspace), or teeny_gemm_f32 for up to 4 rows and
+ * where hipBLASLt does not take the device or shape or the stream is
+ * capturing.  Any M and N; K
  * a multiple of 4; x and w 16-byte aligned. */
 int teeny_linear_f32(const void* x, const void* w, void* y, int M, int N, int K,
                      hipStream_t stream);

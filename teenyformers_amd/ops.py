@@ -174,10 +174,10 @@ def flash_attn2_bwd(q, k, v, o, lse, do, softmax_scale: float | None = None, cau
     B, Hq, Sq, D = q4.shape
     Hkv, Sk = k4.shape[1], k4.shape[2]
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
-    ws_bytes = flash_attn2_bwd_workspace_bytes(q4, k4)
-    if workspace is None:
-        workspace = torch.empty(ws_bytes, dtype=torch.uint8, device=q.device)
     code = _code(q4)
+    if workspace is None:
+        n = _lib.lib().teeny_flash_attn2_bwd_workspace_bytes_shared(Sq, Sk, B, Hq, Hkv, D, code)
+        workspace = torch.empty(n, dtype=torch.uint8, device=q.device)
     gdt = q.dtype
     if grad_f32 and q.dtype == torch.bfloat16:
         code |= _lib.TEENY_GRAD_F32
