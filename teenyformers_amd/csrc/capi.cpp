@@ -11,6 +11,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <atomic>
 #include <cmath>
 #include <cstdint>
@@ -372,6 +373,33 @@ DkdvPlan dkdv_plan(bool causal, int n_ctx_q, int n_ctx_k, int batch, int hq, int
   return p;
 }
 
+// bf16 dK/dV of problems whose 128-key blocks do not fill the device: how many
+// workgroups share the walk of one.  The time is that of the longest walk
+// (items: q heads of the group x 32-row query blocks), so few blocks with long
+// walks are shared until two workgroups per CU run with 12 items each, and to
+// four per CU where 64 items each remain; with more than half a block per CU
+// only walks of 96 items or more gain.  The merge reads every share.  Measured,
+// forward + backward in us, unshared (or in two wavefront groups) against this:
+//   B1 Hq32 Hkv8 S1021 D64 fp32 gradients  153 ->  82   (8 shares)
+//   B1 Hq8 Hkv1 S3125 D128                 634 -> 208   (16)
+//   B1 Hq32 Hkv8 S2048 / S4096 D128        283 -> 227, 684 -> 622   (4)
+//   B1 Hq64 Hkv8 S4096 D128               1352 -> 1187  (4)
+//   B2 Hq32 Hkv8 S1024 D128                182 -> 138   (4)
+//   B2 Hq32 Hkv4 S264 D64 bidirectional     72 ->  42   (6)
+// and where the rule leaves one: B1 H32 S1024 D128 92 (103 with 2), B4 H4 S1090
+// 91 (95), B2 H8 S404 46 (50), B1 H32 S2048 207 (240), B1 Hq64 Hkv8 S8191 4312
+// (4415).
+int dkdv_share(int n_ctx_q, int n_ctx_k, int batch, int hq, int hkv) {
+  const long cus = device_cus();
+  const long wgs = (long)((n_ctx_k + 127) / 128) * batch * hkv;
+  const long items = (long)(hq / hkv) * ((n_ctx_q + 31) / 32);
+  if (2 * wgs > cus && items < 96) return 1;
+  const long s2 = std::min(2 * cus / wgs, items / 12);
+  const long s4 = wgs <= cus ? std::min(4 * cus / wgs, items / 64) : 1;
+  const long s = std::min(std::max(s2, s4), 16L);
+  return s < 2 ? 1 : (int)s;
+}
+
 size_t dkdv_split_bytes(int n_ctx_k, int batch, int hkv, int head_dim, int split) {
   if (split <= 1) return 0;
   return align256(2 * (size_t)split * batch * hkv * n_ctx_k * head_dim * sizeof(float));
@@ -430,6 +458,12 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
     // two-group kernel runs instead, the group being even)
     DkdvPlan plan = dkdv_plan(causal, n_ctx_q, n_ctx_k, batch, hq, hkv, dtype);
     const size_t base = fa2_bwd_ws(n_ctx_q, batch, hq, head_dim, dtype);
+    if (plan.split == 1) {
+      const int share = dkdv_share(n_ctx_q, n_ctx_k, batch, hq, hkv);
+      if (share > 1 &&
+          workspace_bytes >= base + dkdv_split_bytes(n_ctx_k, batch, hkv, head_dim, share))
+        plan = DkdvPlan{1, share};
+    }
     if (plan.split > 1 &&
         workspace_bytes < base + dkdv_split_bytes(n_ctx_k, batch, hkv, head_dim, plan.split))
       plan = DkdvPlan{2, 1};
@@ -693,11 +727,11 @@ size_t teeny_flash_attn2_bwd_workspace_bytes_shared(int n_ctx_q, int n_ctx_k, in
                                                                n_heads_kv, head_dim, dtype);
   if (gqa == 0) return 0;
   dtype &= ~TEENY_GRAD_F32;
-  if (dtype != TEENY_F32) return gqa;
-  const size_t shared =
-      fa2_bwd_ws(n_ctx_q, batch, n_heads_q, head_dim, dtype) +
-      dkdv_split_bytes(n_ctx_k, batch, n_heads_kv, head_dim,
-                       dkdv_f32_split(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv));
+  const int share = dtype == TEENY_F32
+                        ? dkdv_f32_split(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv)
+                        : dkdv_share(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv);
+  const size_t shared = fa2_bwd_ws(n_ctx_q, batch, n_heads_q, head_dim, dtype) +
+                        dkdv_split_bytes(n_ctx_k, batch, n_heads_kv, head_dim, share);
   return shared > gqa ? shared : gqa;
 }
 

@@ -22,9 +22,9 @@
 //      streamed into double-buffered LDS by buffer_load ... lds and read both
 //      row-wise and, through the LDS transpose read, as Q^T / dO^T),
 //      accumulating dK^T and dV^T in registers: the GQA reduction comes for
-//      free.  With few key blocks (long context, one sequence) the group's q
-//      heads are split over 2-4 workgroups whose fp32 partial sums a third
-//      kernel adds in a fixed order.
+//      free.  With few key blocks (long context or small problems) the walk
+//      is shared by several workgroups whose fp32 partial sums a third kernel
+//      adds in a fixed order.
 // Recomputing S and dP in the dQ kernel costs 7 matrix products per tile
 // pair instead of 5; in exchange neither kernel needs dS round trips through
 // LDS, fp32 atomics or a dQ accumulator in HBM (fp32 atomic adds of that dQ
@@ -68,9 +68,9 @@ struct __attribute__((aligned(16))) DkdvSmem {
   float ld[2][2 * BM];    // LSE * log2(e) and Delta of the tile's rows
 };
 
-// hsplit > 1: the q heads of a GQA group are split over hsplit workgroups
-// (more workgroups when few key blocks would leave CUs idle behind the
-// heaviest causal block); each writes its fp32 dK^T, dV^T sums to
+// hsplit > 1: the walk's (q head, query block) items are shared by hsplit
+// workgroups (more workgroups when few key blocks would leave CUs idle behind
+// the heaviest causal block); each writes its fp32 dK^T, dV^T sums to
 // part[2][hsplit][B * Hkv][nk][D] (dK unscaled), merged by fa2_dkdv_merge.
 // NG = 2: the workgroup is two groups of 4 wavefronts (GRP 0 and 1, the
 // kernel branches once on it) on the same 128 keys, each walking half of
@@ -118,8 +118,8 @@ __device__ __forceinline__ void fa2_bwd_dkdv(
   }
   const int kvh = hh / hsplit, hs = hh - kvh * hsplit;
   const int b = kvh / hkv, hk = kvh - b * hkv;
-  const int group = hq / hkv / hsplit / NG;  // q heads walked by this wavefront group
-  const int head0 = hk * (hq / hkv) + (hs * NG + GRP) * group;
+  const int group = hq / hkv / NG;  // q heads whose tiles this wavefront group's walk is part of
+  const int head0 = hk * (hq / hkv) + GRP * group;
   const int n0 = nb * BN;
   const int kw0 = n0 + 32 * wave;  // this wave's first key
   const int mykey = kw0 + l32;
@@ -151,7 +151,11 @@ __device__ __forceinline__ void fa2_bwd_dkdv(
   const int qb_first = CAUSAL ? n0 / BM : 0;
   const int n_qb = nq_pad / BM;
   const int per_head = n_qb > qb_first ? n_qb - qb_first : 0;
-  const int n_iter = group * per_head;
+  // the walk's (head, q-block) items it0 .. it0 + n_iter - 1: share hs of
+  // hsplit (two groups: the whole walk)
+  const int items = group * per_head;
+  const int it0 = NG == 1 ? (int)((long)items * hs / hsplit) : 0;
+  const int n_iter = NG == 1 ? (int)((long)items * (hs + 1) / hsplit) - it0 : items;
 
   // Q / dO tiles: chunk P = i*256 + tid of a tile holds tile chunk swz(P);
   // the swizzle repeats every 256 chunks.  Wave 0 also brings the rows'
@@ -222,7 +226,11 @@ __device__ __forceinline__ void fa2_bwd_dkdv(
   const float sl2 = scale * kLog2e;
 
   int head = 0, qb = qb_first;  // (head, q-block) of the tile in buffer `it & 1`
-  if (n_iter > 0) load_tile(0, qb_first, 0);
+  if (it0 > 0) {
+    head = it0 / per_head;
+    qb += it0 - head * per_head;
+  }
+  if (n_iter > 0) load_tile(head, qb, 0);
   __builtin_amdgcn_s_waitcnt(0);  // V block and the first tile
   __syncthreads();
 
@@ -408,7 +416,7 @@ __device__ __forceinline__ void fa2_bwd_dkdv(
   //      wavefront's area is free ----
   static_assert(sizeof(DkdvSmem<D>) >= 4 * 32 * D * sizeof(float), "tiles fit the LDS block");
   char* etile = reinterpret_cast<char*>(smg) + wave * (32 * D * (int)sizeof(float));
-  if (hsplit > 1) {  // fp32 sums of this workgroup's heads
+  if (hsplit > 1) {  // fp32 sums of this workgroup's share
     const long n_kvh = total_blocks / num_n_blocks / hsplit;
     float* pk = part + (((long)hs * n_kvh + kvh) * nk + kw0) * D;
     float* pv = pk + (long)hsplit * n_kvh * nk * D;

@@ -423,6 +423,41 @@ def test_fa2_bf16_bwd_gqa_split(cuda, grad_f32):
         assert np.all(np.abs(a - b) <= np.abs(a) * tol + 1e-6)
 
 
+@pytest.mark.parametrize("grad_f32", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
+    (1, 8, 2, 421, 421, 128, True),    # GQA: shares of 56 items cross head boundaries
+    (1, 2, 2, 800, 130, 64, False),    # MHA, bidirectional, two key blocks
+    (1, 8, 1, 97, 300, 64, True),      # causal blocks past the last query row: empty shares
+    (1, 4, 1, 2050, 2050, 64, True),   # instead of the two-group kernel, 16 shares
+])
+def test_fa2_bf16_bwd_shared_walk(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32):
+    """dK/dV walks shared by several workgroups (the default workspace) against
+    the unshared kernels (the smaller workspace) and the oracle.  Both sum the
+    same fp32 products in another order: fp32 gradients within 2^-16 of the
+    tensor's largest value, bf16 ones within one rounding more."""
+    q, k, v, do = inputs(61, B, Hq, Hkv, Sq, Sk, D, bf16=True)
+    scale = 1.0 / math.sqrt(D)
+    qd, kd, vd, dod = (dev(t, torch.bfloat16) for t in (q, k, v, do))
+    o, lse = ops.flash_attn2_fwd(qd, kd, vd, scale, causal)
+    n = ops.flash_attn2_bwd_workspace_bytes(qd)
+    shared = ops._lib.lib().teeny_flash_attn2_bwd_workspace_bytes_shared(
+        Sq, Sk, B, Hq, Hkv, D, ops.TEENY_BF16)
+    assert shared > ops.flash_attn2_bwd_workspace_bytes(qd, kd)
+    ws = torch.empty(n, dtype=torch.uint8, device="cuda")
+    a = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, workspace=ws, grad_f32=grad_f32)
+    b = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
+    c = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
+    assert all(torch.equal(x, y) for x, y in zip(b, c))  # deterministic
+    assert torch.equal(a[0], b[0])
+    for x, y in zip(a[1:], b[1:]):
+        x, y = host(x), host(y)
+        tol = 2.0 ** -16 * np.abs(x).max() + (0.0 if grad_f32 else 2.0 ** -7 * np.abs(x))
+        assert np.all(np.abs(x - y) <= tol)
+    want = O.fa2_bwd(q, k, v, host(o), do, host(lse), scale, causal)
+    for name, got, w in zip(("dq", "dk", "dv"), b, want):
+        check_bf16(name, host(got), w)
+
+
 def _random_shapes(n, seed=2026):
     """Seeded random shapes off the tile grid: ragged lengths, Sq != Sk, GQA
     groups 1-8, both head dims."""
