@@ -444,6 +444,17 @@ int teeny_linear_swiglu_sl_bf16(const void* x, const void* w_s, void* y, int M, 
                                 hipStream_t stream);
 int teeny_linear_partials_sl_bf16(const void* x, const void* w_s, float* parts, int M, int N,
                                   int K, int k_split, hipStream_t stream);
+
+/* The streamed products of a decode step of up to 64 sequences, one entry for
+ * all forms: op TEENY_LINEAR_PLAIN (out bf16 [M, N]), TEENY_LINEAR_SWIGLU (w
+ * [2N, K] gate rows then up rows, out bf16 [M, N]) or TEENY_LINEAR_PARTIALS
+ * (out fp32 slabs [n][M][N], as teeny_linear_partials_bf16); layout 0: w
+ * row-major, 1: in the streaming layout.  N a multiple of 128 (64 with SwiGLU),
+ * K of 128; k_split is read by TEENY_LINEAR_PARTIALS only.  Up to 16 rows: the
+ * entries above, the same bits. */
+enum { TEENY_LINEAR_PLAIN = 0, TEENY_LINEAR_SWIGLU = 1, TEENY_LINEAR_PARTIALS = 2 };
+int teeny_linear_rows_bf16(const void* x, const void* w, void* out, int M, int N, int K, int op,
+                           int k_split, int layout, hipStream_t stream);
 int teeny_fused_add_rmsnorm_partials_fwd(const float* parts, int n_parts, const void* residual,
                                          void* y, void* h, float* rstd, const void* weight,
                                          int M, int N, float eps, int dtype,

@@ -14,6 +14,7 @@ LIB_PATH = os.path.join(PKG, "libteeny_hip.so")
 HEADER = os.path.join(os.path.dirname(PKG), "include", "teeny_hip.h")
 
 TEENY_F32, TEENY_BF16, TEENY_I32 = 0, 1, 2
+TEENY_LINEAR_PLAIN, TEENY_LINEAR_SWIGLU, TEENY_LINEAR_PARTIALS = 0, 1, 2
 TEENY_GRAD_F32 = 0x100  # or-ed into a bf16 backward's dtype: fp32 dq/dk/dv
 
 
@@ -88,6 +89,7 @@ _SIGNATURES = {
     "teeny_linear_sl_bf16": ([_p, _p, _p, _i, _i, _i, _p], _i),
     "teeny_linear_swiglu_sl_bf16": ([_p, _p, _p, _i, _i, _i, _p], _i),
     "teeny_linear_partials_sl_bf16": ([_p, _p, _p, _i, _i, _i, _i, _p], _i),
+    "teeny_linear_rows_bf16": ([_p, _p, _p] + [_i] * 6 + [_p], _i),
     "teeny_fused_add_rmsnorm_partials_fwd": ([_p, _i, _p, _p, _p, _p, _p, _i, _i, _f, _i, _p], _i),
     "teeny_qkv_rope_split_partials_dev": ([_p, _i, _p, _p, _p, _i, _i, _p, _i, _i, _i, _i, _f,
                                            _i, _p], _i),

@@ -1171,13 +1171,53 @@ static int linear_sk_check(const void* x, const void* w, const void* y, int M, i
   return TEENY_OK;
 }
 
+// The same kernels for up to 64 rows: tiles of 16 x rows, 1, 2 or 4 of them.
+static int launch_linear_rows(const void* x, const void* w, void* y, int M, int N, int K, int op,
+                              int k_split, int layout, hipStream_t stream) {
+  const char* mt = M <= 16 ? "" : M <= 32 ? "_m2" : "_m4";
+  char name[64];
+  snprintf(name, sizeof name, "teeny_linear_%s_%s%s", layout ? "sl" : "sk",
+           op == TEENY_LINEAR_SWIGLU ? "swiglu_bf16" : op == TEENY_LINEAR_PARTIALS ? "part_bf16"
+                                                                                  : "bf16",
+           mt);
+  void* args[] = {&x, &w, &y, &M, &N, &K, &k_split};  // the last for the K split only
+  const unsigned splits =
+      op == TEENY_LINEAR_PARTIALS ? (unsigned)teeny_linear_partials_count(K, k_split) : 1u;
+  return launch(name, dim3((unsigned)(N / (op == TEENY_LINEAR_SWIGLU ? 64 : 128)), splits),
+                dim3(512), 0, stream, args);
+}
+
+int teeny_linear_rows_bf16(const void* x, const void* w, void* out, int M, int N, int K, int op,
+                           int k_split, int layout, hipStream_t stream) {
+  if (op < TEENY_LINEAR_PLAIN || op > TEENY_LINEAR_PARTIALS || layout < 0 || layout > 1)
+    return TEENY_ERR_INVALID_VALUE;
+  const bool swiglu = op == TEENY_LINEAR_SWIGLU;
+  if (!x || !w || !out) return TEENY_ERR_NULL_POINTER;
+  if (M <= 0 || N <= 0 || K <= 0 || (swiglu ? 2L : 1L) * N * K >= kMaxElems * 2)
+    return TEENY_ERR_INVALID_SHAPE;
+  if (M > 64 || N % (swiglu ? 64 : 128) != 0 || K % 128 != 0) return TEENY_ERR_UNSUPPORTED;
+  if (op == TEENY_LINEAR_PARTIALS) {
+    if (k_split <= 0) return TEENY_ERR_INVALID_VALUE;
+    if (k_split >= K) k_split = K;
+    else if (k_split % 128 != 0) return TEENY_ERR_INVALID_VALUE;  // whole 128-wide K steps
+    const int n = teeny_linear_partials_count(K, k_split);
+    if (n > 65535 || (long)n * M * N >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
+  }
+  return launch_linear_rows(x, w, out, M, N, K, op, k_split, layout, stream);
+}
+
 // This library's matrix-core GEMM (gemm_bf16.hip: 256 x 256 tiles of y, 512
-// threads), any M; N and K multiples of 64.
+// threads), any M; N and K multiples of 64.  Up to 64 rows its N / 256
+// workgroups would leave most CUs idle (N 4096: 16 of 256; K 14336 285 us):
+// those stream w through the decode kernels where they take the shape (one
+// pass: 64 rows, N 4096 K 14336 165).
 int teeny_gemm_bf16(const void* x, const void* w, void* y, int M, int N, int K,
                     hipStream_t stream) {
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
   if (M <= 0 || N <= 0 || K <= 0 || (long)N * K >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
   if (N % 64 != 0 || K % 64 != 0) return TEENY_ERR_UNSUPPORTED;
+  if (M <= 64 && N % 128 == 0 && K % 128 == 0)
+    return launch_linear_rows(x, w, y, M, N, K, TEENY_LINEAR_PLAIN, K, 0, stream);
   // a workgroup addresses its 256 rows of x and of w with 32-bit byte offsets
   if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
@@ -1253,17 +1293,15 @@ int teeny_linear_f32(const void* x, const void* w, void* y, int M, int N, int K,
   return teeny_gemm_f32(x, w, y, M, N, K, stream);
 }
 
-// Any M, as teeny_linear_bf16: up to 16 rows through linear_bf16.hip's
+// Any M, as teeny_linear_bf16: up to 64 rows through linear_bf16.hip's
 // weight-streaming kernel when F % 64 and K % 128 are 0; otherwise the GEMM
 // with the SwiGLU epilogue (256 rows x 128 features per workgroup).
 int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F, int K,
                              hipStream_t stream) {
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
   if (M <= 0 || F <= 0 || K <= 0 || 2L * F * K >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
-  if (M <= 16 && F % 64 == 0 && K % 128 == 0) {
-    void* args[] = {&x, &w, &y, &M, &F, &K};
-    return launch("teeny_linear_sk_swiglu_bf16", dim3(F / 64), dim3(512), 0, stream, args);
-  }
+  if (M <= 64 && F % 64 == 0 && K % 128 == 0)
+    return launch_linear_rows(x, w, y, M, F, K, TEENY_LINEAR_SWIGLU, K, 0, stream);
   if (F % 32 != 0 || K % 64 != 0) return TEENY_ERR_UNSUPPORTED;
   if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   int tiles_m = (M + 255) / 256, tiles_n = (F + 127) / 128;

@@ -1,9 +1,9 @@
 // Skinny linear layers of a decode step: y[M, N] = x[M, K] . W[N, K]^T with
-// M <= 16 (one new token per sequence), bf16 in, fp32 accumulation.
+// M <= 64 (one new token per sequence), bf16 in, fp32 accumulation.
 //
 // Reference: sym_linear (src/layers/mod.rs:54-58) lowers to the external
 // teeny-core Linear, y = x W^T with W in HF [out, in] layout
-// (src/loader.rs:19-27).  With M <= 16 the product is bound by streaming W
+// (src/loader.rs:19-27).  With so few rows the product is bound by streaming W
 // from HBM once.
 //
 // A workgroup of 8 wavefronts owns 128 output features (16 W rows per
@@ -61,10 +61,11 @@ enum SkMode { SK_BF16, SK_SWIGLU, SK_PART };
 // order are the same, so are the results.
 // PF: the next chunk's W is loaded into a second register set before this
 // chunk's products, and the x barrier leaves those loads in flight.
-template <SkMode MODE, bool SL, bool PF>
+// MT: tiles of 16 x rows, all multiplied by each W fragment.
+template <SkMode MODE, bool SL, bool PF, int MT = 1>
 __device__ __forceinline__ void linear_sk(const bf16* __restrict__ x, const bf16* __restrict__ w,
                                           void* __restrict__ out, int M, int N, int K, int KC) {
-  __shared__ __attribute__((aligned(16))) char xs[2][16 * XS];
+  __shared__ __attribute__((aligned(16))) char xs[2][16 * MT * XS];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r = lane & 15, g = lane >> 4;
@@ -87,7 +88,7 @@ __device__ __forceinline__ void linear_sk(const bf16* __restrict__ x, const bf16
 
   // x staging: a chunk row is 64 16-byte pieces (16 per 128-wide step);
   // thread t copies pieces P = t % TP + TP j of row t / TP
-  constexpr int TP = NW * 64 / 16, XJ = 64 / TP;
+  constexpr int TP = NW * 64 / (16 * MT), XJ = 64 / TP;
   const int xm = tid / TP, xp = tid % TP;
   const bf16* xsrc = x + (long)min(xm, M - 1) * K + 8 * xp;
   u32x4 xv[XJ];
@@ -148,13 +149,17 @@ __device__ __forceinline__ void linear_sk(const bf16* __restrict__ x, const bf16
     const char* xb = xs[(C) & 1] + r * XS + xoff;                                              \
     _Pragma("unroll") for (int j = 0; j < 4; ++j) if (j < ns)                                  \
       _Pragma("unroll") for (int q = 0; q < 4; ++q)                                            \
-        acc = mfma16(A[j][q], *reinterpret_cast<const u32x4*>(xb + xro(j, q)), acc);           \
+        _Pragma("unroll") for (int m = 0; m < MT; ++m)                                         \
+          acc[m] = mfma16(A[j][q], *reinterpret_cast<const u32x4*>(xb + 16 * m * XS + xro(j, q)), \
+                          acc[m]);                                                             \
     if ((C) + 1 < nch) xstore(((C) + 1) & 1, steps_of(k0 + XC));                               \
   } while (0)
 
   xload(kb, steps_of(kb));
   xstore(0, steps_of(kb));
-  f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+  f32x4 acc[MT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m) acc[m] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
   u32x4 a0[4][4], a1[4][4];
   if constexpr (PF) {
     TEENY_SK_WLOAD(a0, kb, steps_of(kb));
@@ -170,31 +175,40 @@ __device__ __forceinline__ void linear_sk(const bf16* __restrict__ x, const bf16
 #undef TEENY_SK_CHUNK
 #undef TEENY_SK_WLOAD
 
-  // lane: token r, features f0 + 4 g + i of the wavefront's 16
+  // lane: tokens 16 m + r, features f0 + 4 g + i of the wavefront's 16
   if constexpr (MODE == SK_SWIGLU) {
     __syncthreads();  // done with xs: reuse it for the up halves
     f32x4* up = reinterpret_cast<f32x4*>(xs[0]);
-    if (wave >= NW / 2) up[(wave - NW / 2) * 64 + lane] = acc;
-    __syncthreads();
-    if (wave < NW / 2 && r < M) {
-      const f32x4 u = up[wave * 64 + lane];
-      float o[4];
+    if (wave >= NW / 2)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float gate = (float)(bf16)acc[i], upv = (float)(bf16)u[i];
-        o[i] = gate * (1.0f / (1.0f + expf(-gate))) * upv;
+      for (int m = 0; m < MT; ++m) up[((wave - NW / 2) * MT + m) * 64 + lane] = acc[m];
+    __syncthreads();
+    if (wave < NW / 2)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) {
+        if (16 * m + r >= M) continue;
+        const f32x4 u = up[(wave * MT + m) * 64 + lane];
+        float o[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          const float gate = (float)(bf16)acc[m][i], upv = (float)(bf16)u[i];
+          o[i] = gate * (1.0f / (1.0f + expf(-gate))) * upv;
+        }
+        bf16* y = (bf16*)out + (long)(16 * m + r) * N + blockIdx.x * (8 * NW) + 16 * wave + 4 * g;
+        *reinterpret_cast<u32x2*>(y) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
       }
-      bf16* y = (bf16*)out + (long)r * N + blockIdx.x * (8 * NW) + 16 * wave + 4 * g;
-      *reinterpret_cast<u32x2*>(y) = u32x2{pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
-    }
-  } else if (r < M) {
-    if constexpr (MODE == SK_BF16) {
-      bf16* y = (bf16*)out + (long)r * N + row0 + 4 * g;
-      *reinterpret_cast<u32x2*>(y) =
-          u32x2{pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3])};
-    } else {
-      float* p = (float*)out + ((long)blockIdx.y * M + r) * N + row0 + 4 * g;
-      *reinterpret_cast<f32x4*>(p) = acc;
+  } else {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      if (16 * m + r >= M) continue;
+      if constexpr (MODE == SK_BF16) {
+        bf16* y = (bf16*)out + (long)(16 * m + r) * N + row0 + 4 * g;
+        *reinterpret_cast<u32x2*>(y) =
+            u32x2{pack_bf16x2(acc[m][0], acc[m][1]), pack_bf16x2(acc[m][2], acc[m][3])};
+      } else {
+        float* p = (float*)out + ((long)blockIdx.y * M + 16 * m + r) * N + row0 + 4 * g;
+        *reinterpret_cast<f32x4*>(p) = acc[m];
+      }
     }
   }
 }
@@ -234,6 +248,42 @@ extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sl_part_bf16(
     const bf16* x, const bf16* w, float* part, int M, int N, int K, int KC) {
   linear_sk<SK_PART, true, false>(x, w, part, M, N, K, KC);
 }
+
+// Decode steps of 17 to 64 sequences: the same kernels with 2 or 4 tiles of 16
+// x rows (MT), each W fragment multiplied by all of them; x then takes 65 or
+// 130 KiB of LDS, so one or two workgroups per CU.  One chunk of W in flight:
+// the look-ahead of the 16-row forms was 2-26 % slower here.  From HBM, 64
+// rows, streaming layout (row-major in brackets), against the 256 x 256 GEMM
+// tiles they replace: gate_up 28672 x 4096 with SwiGLU 52 us (58) against 94,
+// 128256 x 4096 200 us (218), K-split 4096 x 14336 27 us against 285, 6144 x
+// 4096 16 us against 79.
+#define TEENY_SK_ROWS(MT)                                                                       \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sk_bf16_m##MT(            \
+      const bf16* x, const bf16* w, bf16* y, int M, int N, int K) {                             \
+    linear_sk<SK_BF16, false, false, MT>(x, w, y, M, N, K, K);                                  \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sk_swiglu_bf16_m##MT(     \
+      const bf16* x, const bf16* w, bf16* y, int M, int F, int K) {                             \
+    linear_sk<SK_SWIGLU, false, false, MT>(x, w, y, M, F, K, K);                                \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sk_part_bf16_m##MT(       \
+      const bf16* x, const bf16* w, float* part, int M, int N, int K, int KC) {                 \
+    linear_sk<SK_PART, false, false, MT>(x, w, part, M, N, K, KC);                              \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sl_bf16_m##MT(            \
+      const bf16* x, const bf16* w, bf16* y, int M, int N, int K) {                             \
+    linear_sk<SK_BF16, true, false, MT>(x, w, y, M, N, K, K);                                   \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sl_swiglu_bf16_m##MT(     \
+      const bf16* x, const bf16* w, bf16* y, int M, int F, int K) {                             \
+    linear_sk<SK_SWIGLU, true, false, MT>(x, w, y, M, F, K, K);                                 \
+  }                                                                                             \
+  extern "C" __global__ __launch_bounds__(NW * 64) void teeny_linear_sl_part_bf16_m##MT(       \
+      const bf16* x, const bf16* w, float* part, int M, int N, int K, int KC) {                 \
+    linear_sk<SK_PART, true, false, MT>(x, w, part, M, N, K, KC);                               \
+  }
+TEENY_SK_ROWS(2)
+TEENY_SK_ROWS(4)
 
 // Row-major W [N, K] -> the streaming layout [N/16][K/128][q][g][r][8]:
 // piece p = (((nb * K/128 + ks) * 4 + q) * 4 + g) * 16 + r holds

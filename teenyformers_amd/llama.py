@@ -23,12 +23,13 @@ MI355X-specific structure (same arithmetic):
   * Linear layers (teeny-core's external `Linear`, src/layers/mod.rs:54-58,
     y = x W^T with W [out, in]) run through the library's linear entry
     points: a prompt's products through hipBLASLt (teeny_linear_bf16 /
-    teeny_linear_f32), and with at most 16 rows (a decode step) the
-    weight-streaming kernels: gate_up fused with SwiGLU, and q|k|v, o and
-    down split over K into fp32 slabs that the QKV split and the
-    residual-add norms sum.  Decode steps of more than 16 sequences run the
-    library's own GEMM (ops.own_gemm), the kernel a captured graph runs, so
-    eager and graph-replayed steps compute the same bits.
+    teeny_linear_f32), and with at most 16 rows, or in a decode step of at
+    most 64 sequences, the weight-streaming kernels: gate_up fused with
+    SwiGLU, and q|k|v, o and down split over K into fp32 slabs that the QKV
+    split and the residual-add norms sum.  Decode steps of more sequences
+    run the library's own GEMM.  Decode steps run within ops.own_gemm, the
+    kernels a captured graph runs, so eager and graph-replayed steps compute
+    the same bits.
 """
 from __future__ import annotations
 
@@ -216,13 +217,14 @@ class Llama:
         Hq, Hkv, D = cfg.n_heads, cfg.n_kv_heads(), cfg.head_dim()
         p = f"model.layers.{i}.self_attn."
         # [B, S, (Hq+2Hkv) D]; K-split fp32 slabs at decode sizes
-        qkv = ops.linear_split(n1, self._lw(p + "qkv_proj.weight"))
+        rows = ops.split_rows()
+        qkv = ops.linear_split(n1, self._lw(p + "qkv_proj.weight"), rows=rows)
         scale = cfg.softmax_scale()
         if isinstance(pos0, torch.Tensor) and self._fused_decode(qkv, cache):
             # one launch: QKV split, RoPE, cache write and attention
             o = ops.decode_qkv_attention(qkv, cache.k[i], cache.v[i], pos0, Hq, Hkv,
                                          cfg.rope_base, scale)
-            return ops.linear_split(o.view(B, 1, Hq * D), self._lw(p + "o_proj.weight"))
+            return ops.linear_split(o.view(B, 1, Hq * D), self._lw(p + "o_proj.weight"), rows=rows)
         if (not isinstance(pos0, torch.Tensor) and pos0 == 0
                 and not isinstance(qkv, ops.Partials) and qkv.dtype == torch.bfloat16):
             # bf16 prompt: K and V into the cache; the attention reads the q
@@ -258,7 +260,7 @@ class Llama:
             o, _ = ops.flash_attn2_fwd(q, cache.k[i], cache.v[i], scale, causal=True)
         # one position: [B, Hq, 1, D] is already the merged [B, 1, Hq D] layout
         att = o.view(B, S, Hq * D) if S == 1 else ops.merge_heads(o)
-        return ops.linear_split(att, self._lw(p + "o_proj.weight"))
+        return ops.linear_split(att, self._lw(p + "o_proj.weight"), rows=rows)
 
     def _rope_table(self, n: int, device) -> torch.Tensor:
         """RoPE's (cos, sin) for positions 0 .. n-1 at least (kept, grown to
@@ -290,7 +292,7 @@ class Llama:
         """src/layers/ffn.rs:47-56."""
         p = f"model.layers.{i}.mlp."
         f = ops.linear_swiglu(n2, self._lw(p + "gate_up_proj.weight"))
-        return ops.linear_split(f, self._lw(p + "down_proj.weight"))
+        return ops.linear_split(f, self._lw(p + "down_proj.weight"), rows=ops.split_rows())
 
     def hidden(self, ids: torch.Tensor, cache: KVCache, pos0, trace: list | None = None
                ) -> torch.Tensor:
@@ -451,8 +453,8 @@ class DecodeGraph:
 
     def _step(self, trace: list | None = None):
         m = self.model
-        # the eager first step runs the kernels the capture records (above 16
-        # sequences the library's own GEMM, as teeny_linear_bf16 under capture)
+        # the eager first step runs the kernels the capture records (the
+        # library's own at any batch, as teeny_linear_bf16 under capture)
         with ops.own_gemm():
             h = m.hidden(self.ids, self.cache, self.pos, trace=trace)
             self.logits = m.logits(h[:, -1])

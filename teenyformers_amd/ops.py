@@ -542,11 +542,15 @@ def _no_grad(x2: torch.Tensor, w: torch.Tensor) -> bool:
     return not (torch.is_grad_enabled() and (x2.requires_grad or w.requires_grad))
 
 
-def _skinny(x2: torch.Tensor, w: torch.Tensor, n_out: int, row_tile: int = 128) -> bool:
-    """Shapes the decode-step linear kernels take."""
+def _skinny(x2: torch.Tensor, w: torch.Tensor, n_out: int, row_tile: int = 128,
+            rows: int | None = None) -> bool:
+    """Shapes the decode-step linear kernels take: up to 16 rows, and up to 64
+    within own_gemm() (other products of 17 rows or more go to hipBLASLt)."""
     M, K = x2.shape
+    if rows is None:
+        rows = split_rows()
     return (_no_grad(x2, w) and x2.dtype == torch.bfloat16 and w.dtype == torch.bfloat16
-            and x2.is_cuda and 1 <= M <= 16 and K % 128 == 0 and n_out % row_tile == 0
+            and x2.is_cuda and 1 <= M <= rows and K % 128 == 0 and n_out % row_tile == 0
             and w.is_contiguous())
 
 
@@ -569,8 +573,8 @@ _own_gemm = threading.local()
 @contextlib.contextmanager
 def own_gemm():
     """Within this block, products run this library's GEMMs instead of
-    hipBLASLt: bf16 products of more than 16 rows teeny_gemm_bf16, fp32
-    products teeny_gemm_f32.  That is the rule a captured graph follows by
+    hipBLASLt: bf16 products of 17 to 64 rows the weight-streaming decode
+    kernels, of more rows teeny_gemm_bf16, fp32 products teeny_gemm_f32.  That is the rule a captured graph follows by
     itself (the linear entry points never run hipBLASLt under capture),
     applied to eager calls so that an eager step and its graph replay run
     the same kernels."""
@@ -582,13 +586,19 @@ def own_gemm():
         _own_gemm.on = prev
 
 
+def split_rows() -> int:
+    """The row count up to which a model's products are taken as linear_split's
+    Partials: 64 within own_gemm() (decode steps), 16 otherwise (short prompts)."""
+    return 64 if getattr(_own_gemm, "on", False) else 16
+
+
 class StreamWeight:
     """A bf16 weight W [N, K] with its streaming-layout copy
     (teeny_linear_stream_layout_bf16: the order in which the decode-step
     kernels load it, one contiguous KiB per load instruction).  linear,
     linear_swiglu and linear_split take it in place of the tensor: products
-    of up to 16 rows read the copy (teeny_linear_*sl_bf16, the same outputs),
-    other products the row-major W.  Costs one more copy of W.  The copy is
+    of up to 16 rows (64 in a decode step) read the copy, with the same
+    outputs, other products the row-major W.  Costs one more copy of W.  The copy is
     made once, here: after an in-place change of W, make a new StreamWeight."""
 
     def __init__(self, w: torch.Tensor):
@@ -625,7 +635,8 @@ def linear(x: torch.Tensor, w) -> torch.Tensor:
         if _skinny(x2, w.w, N):
             x2 = x2.contiguous()
             y = torch.empty((x2.shape[0], N), dtype=x.dtype, device=x.device)
-            call("teeny_linear_sl_bf16", _p(x2), _p(w.s), _p(y), x2.shape[0], N, K, _stream())
+            call("teeny_linear_rows_bf16", _p(x2), _p(w.s), _p(y), x2.shape[0], N, K,
+                 _lib.TEENY_LINEAR_PLAIN, K, 1, _stream())
             return y.view(*x.shape[:-1], N)
         w = w.w
     if _gemm_f32(x2, w):
@@ -686,11 +697,9 @@ def linear_swiglu(x: torch.Tensor, w_gate_up) -> torch.Tensor:
         return swiglu(linear(x, w))
     x2 = x2.contiguous()
     y = torch.empty((x2.shape[0], F), dtype=x.dtype, device=x.device)
-    if isinstance(w_gate_up, StreamWeight):
-        call("teeny_linear_swiglu_sl_bf16", _p(x2), _p(w_gate_up.s), _p(y), x2.shape[0], F, K,
-             _stream())
-    else:
-        call("teeny_linear_swiglu_bf16", _p(x2), _p(w), _p(y), x2.shape[0], F, K, _stream())
+    streamed = isinstance(w_gate_up, StreamWeight)
+    call("teeny_linear_rows_bf16", _p(x2), _p(w_gate_up.s if streamed else w), _p(y), x2.shape[0], F,
+         K, _lib.TEENY_LINEAR_SWIGLU, K, int(streamed), _stream())
     return y.view(*x.shape[:-1], F)
 
 
@@ -722,25 +731,22 @@ def _k_split(K: int, N: int) -> int:
     return -(-steps // best) * 128
 
 
-def linear_split(x: torch.Tensor, w, k_split: int | None = None):
-    """x w^T as Partials where the decode kernels take the shape (up to 16
-    bf16 rows), else the GEMM's tensor.  k_split (a multiple of 128) sets K
+def linear_split(x: torch.Tensor, w, k_split: int | None = None, rows: int = 16):
+    """x w^T as Partials where the decode kernels take the shape (up to `rows`
+    bf16 rows, at most 64), else the GEMM's tensor.  k_split (a multiple of 128) sets K
     per slab; by default it is chosen to spread the work over the CUs.  w may
     be a StreamWeight."""
     x2 = x.reshape(-1, x.shape[-1])
     N, K = w.shape
     if K != x2.shape[1]:
         raise ValueError(f"linear: x has {x2.shape[1]} features, w expects {K}")
-    if not _skinny(x2, _row_major(w), N):
+    if not _skinny(x2, _row_major(w), N, rows=min(rows, 64)):
         return linear(x, _row_major(w))
     x2 = x2.contiguous()
     ks = _k_split(K, N) if k_split is None else k_split
     n = _lib.lib().teeny_linear_partials_count(K, ks)
     slabs = torch.empty((n, x2.shape[0], N), dtype=torch.float32, device=x.device)
-    if isinstance(w, StreamWeight):
-        call("teeny_linear_partials_sl_bf16", _p(x2), _p(w.s), _p(slabs), x2.shape[0], N, K, ks,
-             _stream())
-    else:
-        call("teeny_linear_partials_bf16", _p(x2), _p(w), _p(slabs), x2.shape[0], N, K, ks,
-             _stream())
+    streamed = isinstance(w, StreamWeight)
+    call("teeny_linear_rows_bf16", _p(x2), _p(w.s if streamed else w), _p(slabs), x2.shape[0], N, K,
+         _lib.TEENY_LINEAR_PARTIALS, ks, int(streamed), _stream())
     return Partials(slabs, (*x.shape[:-1], N), x.dtype)

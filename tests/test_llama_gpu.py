@@ -424,6 +424,31 @@ def _seq_sum_bf16(slabs):
     return O.bf16_round(acc)
 
 
+@pytest.mark.parametrize("M", [17, 32, 33, 64])
+@pytest.mark.parametrize("N,K", [(128, 128), (256, 640), (384, 1536)])  # K off the 512-wide chunks
+def test_linear_rows_17_to_64(cuda, M, N, K):
+    """Decode products of 17 to 64 rows (2 and 4 tiles of x rows): each form
+    and layout against float64 (fp32 sums: |err| <= 2 K u sum|x w|, then one
+    bf16 rounding of 2^-9), the layouts bit-equal, and the first 16 rows
+    bit-equal to the 16-row kernels."""
+    x, w = _bf16_dev(np.random.default_rng(M).standard_normal((M, K)).astype(np.float32)), \
+        _bf16_dev((0.05 * np.random.default_rng(N).standard_normal((N, K))).astype(np.float32))
+    sw = ops.StreamWeight(w)
+    want, mag = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    bound = 2 * K * 2.0 ** -24 * mag
+    with ops.own_gemm():
+        y, ys = ops.linear(x, w), ops.linear(x, sw)
+        f, fs = ops.linear_swiglu(x, w), ops.linear_swiglu(x, sw)
+        p, ps = ops.linear_split(x, w, 128, rows=64), ops.linear_split(x, sw, 128, rows=64)
+    assert torch.equal(y, ys) and torch.equal(f, fs) and torch.equal(p.slabs, ps.slabs)
+    assert torch.equal(y[:16], ops.linear(x[:16], w))
+    assert torch.equal(f[:16], ops.linear_swiglu(x[:16], w))
+    assert torch.equal(p.slabs[:, :16], ops.linear_split(x[:16], w, 128).slabs)
+    assert bool(((y.double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all())
+    assert bool(((p.slabs.double().sum(0) - want).abs() <= bound).all())
+    assert torch.equal(f, ops.swiglu(y))
+
+
 @pytest.mark.parametrize("d,k_split", [
     (2048, None), (2048, 384), (2048, 128),  # 16, 6 (a last group of 6) and 16 slabs
     (4096, 640), (8192, 1152)])              # 7 and 8 slabs of 2 and 4 chunks per thread
