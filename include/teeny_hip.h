@@ -481,6 +481,21 @@ int teeny_decode_qkv_attention_dev(const float* parts, int n_parts, void* k_cach
                                    int n_heads_kv, int head_dim, int cache_len,
                                    const int32_t* n_past, float ln_rope_base,
                                    float softmax_scale, int dtype, hipStream_t stream);
+/* The same with each (b, kv head)'s keys shared by n_split workgroups, whose
+ * partials (in the workspace) a second kernel merges: for long caches and few
+ * sequences.  teeny_decode_qkv_attention_splits gives the measured choice, 1
+ * where the one-launch form above is faster; the workspace is
+ * teeny_decode_qkv_attention_workspace_bytes (0 for one split). */
+int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len);
+size_t teeny_decode_qkv_attention_workspace_bytes(int batch, int n_heads_q, int head_dim,
+                                                  int n_split);
+int teeny_decode_qkv_attention_split_dev(const float* parts, int n_parts, void* k_cache,
+                                         void* v_cache, void* o, int batch, int n_heads_q,
+                                         int n_heads_kv, int head_dim, int cache_len,
+                                         const int32_t* n_past, float ln_rope_base,
+                                         float softmax_scale, int dtype, int n_split,
+                                         void* workspace, size_t workspace_bytes,
+                                         hipStream_t stream);
 
 #ifdef __cplusplus
 }

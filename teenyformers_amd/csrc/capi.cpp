@@ -1029,11 +1029,49 @@ int teeny_qkv_rope_split_partials_dev(const float* parts, int n_parts, void* q_o
                 dim3(256), shmem, stream, args);
 }
 
+// Workgroups that share the keys of a (b, kv head) in the one-launch decode
+// attention: a key tile (32) per wavefront at full cache at the finest, until
+// every CU has a workgroup, at most 16 (32 was 0-50 % slower than 16).
+// Measured in a graph, 32 q and 8 kv heads of 128, us unsplit against this:
+// one sequence 1001 of 1100 keys 11.5 -> 10.5, 3901 of 4096 26.4 -> 11.7,
+// 12001 of 12200 111 -> 18.5 (30 through the unfused kernels); 8 sequences
+// 3901 of 4096 47.5 -> 31.9; an almost empty long cache (501 of 4096) 8.1 ->
+// 9.9, the merge's launch.  Up to 1024 rows and from half the CUs' worth of
+// (b, kv head) pairs it does not pay (16 sequences, 1001 of 1200: 18.2, 20.1
+// with 2; 640 rows, one sequence: 9.2, 9.8 with 4).
+int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len) {
+  if (batch <= 0 || n_heads_kv <= 0 || cache_len <= 0) return 0;
+  const long wgs = (long)batch * n_heads_kv;
+  if (cache_len <= 1024 || 2 * wgs >= device_cus()) return 1;
+  const long s = std::min((long)device_cus() / wgs, (long)(cache_len + 255) / 256);
+  return s < 2 ? 1 : s > 16 ? 16 : (int)s;
+}
+
+size_t teeny_decode_qkv_attention_workspace_bytes(int batch, int n_heads_q, int head_dim,
+                                                  int n_split) {
+  if (batch <= 0 || n_heads_q <= 0 || head_dim <= 0 || n_split <= 1) return 0;
+  const size_t rows = (size_t)batch * n_heads_q * n_split;
+  return 2 * align256(rows * sizeof(float)) + align256(rows * head_dim * sizeof(float));
+}
+
 int teeny_decode_qkv_attention_dev(const float* parts, int n_parts, void* k_cache,
                                    void* v_cache, void* o, int batch, int n_heads_q,
                                    int n_heads_kv, int head_dim, int cache_len,
                                    const int32_t* n_past, float ln_rope_base,
                                    float softmax_scale, int dtype, hipStream_t stream) {
+  return teeny_decode_qkv_attention_split_dev(parts, n_parts, k_cache, v_cache, o, batch, n_heads_q,
+                                              n_heads_kv, head_dim, cache_len, n_past,
+                                              ln_rope_base, softmax_scale, dtype, 1, nullptr, 0,
+                                              stream);
+}
+
+int teeny_decode_qkv_attention_split_dev(const float* parts, int n_parts, void* k_cache,
+                                   void* v_cache, void* o, int batch, int n_heads_q,
+                                   int n_heads_kv, int head_dim, int cache_len,
+                                   const int32_t* n_past, float ln_rope_base,
+                                   float softmax_scale, int dtype, int n_split, void* workspace,
+                                   size_t workspace_bytes, hipStream_t stream) {
+  int rc;
   if (!parts || !k_cache || !v_cache || !o || !n_past) return TEENY_ERR_NULL_POINTER;
   if (dtype != TEENY_BF16 || (head_dim != 64 && head_dim != 128)) return TEENY_ERR_UNSUPPORTED;
   if (n_parts <= 0 || batch <= 0 || n_heads_q <= 0 || n_heads_kv <= 0 || cache_len <= 0 ||
@@ -1050,12 +1088,28 @@ int teeny_decode_qkv_attention_dev(const float* parts, int n_parts, void* k_cach
     return TEENY_ERR_INVALID_SHAPE;
   if (!std::isfinite(ln_rope_base) || !scale_ok(softmax_scale, dtype))
     return TEENY_ERR_INVALID_VALUE;
+  if (n_split < 1 || n_split > 65535) return TEENY_ERR_INVALID_VALUE;
+  float *pm = nullptr, *pl = nullptr, *po = nullptr;
+  if (n_split > 1) {
+    if (!workspace || workspace_bytes < teeny_decode_qkv_attention_workspace_bytes(
+                                            batch, n_heads_q, head_dim, n_split))
+      return TEENY_ERR_WORKSPACE;
+    const size_t rows = (size_t)batch * n_heads_q * n_split;
+    pm = (float*)workspace;
+    pl = (float*)((char*)workspace + align256(rows * sizeof(float)));
+    po = (float*)((char*)workspace + 2 * align256(rows * sizeof(float)));
+  }
   char name[48];
   snprintf(name, sizeof name, "teeny_decode_qkv_attn_bf16_d%d", head_dim);
   void* args[] = {&parts,      &n_parts,   &part_stride, &k_cache,      &v_cache,
                   &o,          &n_heads_q, &n_heads_kv,  &n_past,       &cache_len,
-                  &ln_rope_base, &softmax_scale};
-  return launch(name, dim3((unsigned)(batch * n_heads_kv)), dim3(512), 0, stream, args);
+                  &ln_rope_base, &softmax_scale, &pm,    &pl,           &po};
+  rc = launch(name, dim3((unsigned)(batch * n_heads_kv), (unsigned)n_split), dim3(512), 0, stream,
+              args);
+  if (rc || n_split == 1) return rc;
+  void* a1[] = {&pm, &pl, &po, &o, &n_split, &head_dim};
+  return launch("teeny_decode_attn_combine_bf16", dim3((unsigned)(batch * n_heads_q)),
+                dim3(head_dim), 0, stream, a1);
 }
 
 // matrix-core kernels: keys per wavefront chosen so that one step runs

@@ -197,6 +197,10 @@ __device__ void decode_mfma(const bf16* __restrict__ q, const bf16* __restrict__
 //   3. the 8 partials (max, sum, unnormalised O) are merged in LDS and
 //      o [B, Hq, D] is stored, and the new k, v row is written to the cache
 //      (row n_past, when it is below cache_len) for the next steps.
+// gridDim.y > 1 (long caches, few sequences: B * Hkv workgroups would leave
+// most CUs idle): the keys are shared by that many such workgroups of a
+// (b, kv head), each repeating step 1, and the partials go to pm, pl, po for
+// teeny_decode_attn_combine (the host's rule and its figures: capi.cpp).
 // It replaces the QKV split, the split-K decode kernel and the combine
 // kernel of the unfused path with one launch and no partials in HBM.
 constexpr int kDqWaves = 8;
@@ -224,7 +228,8 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
                                 bf16* __restrict__ kc, bf16* __restrict__ vc,
                                 bf16* __restrict__ o, int hq, int hkv,
                                 const int* __restrict__ n_past, int cache_len, float ln_base,
-                                float scale) {
+                                float scale, float* __restrict__ pm, float* __restrict__ pl,
+                                float* __restrict__ po) {
   constexpr int DC = D / 16, DT = D / 32, CPR = D / 8;
   constexpr int TILE = TK * D * 2;  // bytes of a K or V tile
   constexpr int NLD = TILE / 1024;  // 16-byte-per-lane loads per tile
@@ -240,8 +245,10 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
   const int n_keys = __builtin_amdgcn_readfirstlane(min(pos + 1, cache_len));
 
   // this wavefront's keys k0 .. k1 - 1, in 32-key tiles through its LDS buffer
-  const int kpw = ((n_keys + kDqWaves - 1) / kDqWaves + TK - 1) / TK * TK;
-  const int k0 = wave * kpw;
+  const int n_split = gridDim.y, split = blockIdx.y;
+  const int waves = kDqWaves * n_split;  // that share the keys
+  const int kpw = ((n_keys + waves - 1) / waves + TK - 1) / TK * TK;
+  const int k0 = (split * kDqWaves + wave) * kpw;
   const int k1 = min(k0 + kpw, n_keys);
   const int n_tiles = k0 < k1 ? (k1 - k0 + TK - 1) / TK : 0;
   // the cache up to row pos - 1 (the rows this step reads from it); rows at
@@ -450,17 +457,28 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
     float mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kDqWaves; ++w) mm = fmaxf(mm, sm.u.c.m[w][hh]);
+    const float ref = mm == -INFINITY ? 0.0f : mm;  // a split may have no keys
     float num = 0.0f, den = 0.0f;
 #pragma unroll
     for (int w = 0; w < kDqWaves; ++w) {
-      const float e = fast_exp2(sm.u.c.m[w][hh] - mm);  // 0 for a wavefront without keys
+      const float e = fast_exp2(sm.u.c.m[w][hh] - ref);  // 0 for a wavefront without keys
       num += e * sm.u.c.o[w][hh * D + d];
       den += e * sm.u.c.l[w][hh];
     }
-    o[((long)b * hq + hk * group + hh) * D + d] = (bf16)(num / den);
+    const long row = (long)b * hq + hk * group + hh;
+    if (n_split == 1) {
+      o[row * D + d] = (bf16)(num / den);
+    } else {
+      const long r = row * n_split + split;
+      po[r * D + d] = num;
+      if (d == 0) {
+        pm[r] = mm * kLn2;  // natural-log units for the merge; -inf without keys
+        pl[r] = den;
+      }
+    }
   }
   // the new k, v row to the cache, for the next steps
-  if (pos >= 0 && pos < cache_len && tid < 2 * CPR) {
+  if (split == 0 && pos >= 0 && pos < cache_len && tid < 2 * CPR) {
     const int c = tid % CPR;
     bf16* cache = tid < CPR ? kc : vc;
     *reinterpret_cast<u32x4*>(cache + ((long)kvh * cache_len + pos) * D + 8 * c) =
@@ -485,9 +503,10 @@ TEENY_DECODE_BF16_INST(128)
 #define TEENY_DECODE_QKV_INST(D)                                                                 \
   extern "C" __global__ __launch_bounds__(512) void teeny_decode_qkv_attn_bf16_d##D(            \
       const float* parts, int n_parts, long part_stride, bf16* kc, bf16* vc, bf16* o, int hq,    \
-      int hkv, const int* n_past, int cache_len, float ln_base, float scale) {                   \
+      int hkv, const int* n_past, int cache_len, float ln_base, float scale, float* pm,          \
+      float* pl, float* po) {                                                                    \
     decode_qkv_attn<D>(parts, n_parts, part_stride, kc, vc, o, hq, hkv, n_past, cache_len,      \
-                       ln_base, scale);                                                          \
+                       ln_base, scale, pm, pl, po);                                              \
   }
 
 TEENY_DECODE_QKV_INST(64)

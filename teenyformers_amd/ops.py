@@ -498,10 +498,16 @@ def decode_attention(q, k_cache, v_cache, n_keys: int, softmax_scale: float | No
     return out
 
 
+def decode_qkv_splits(batch: int, n_heads_kv: int, cache_len: int) -> int:
+    """How many workgroups share each (b, kv head)'s keys in decode_qkv_attention."""
+    return _lib.lib().teeny_decode_qkv_attention_splits(batch, n_heads_kv, cache_len)
+
+
 def decode_qkv_attention(qkv: "Partials", k_cache, v_cache, n_past, n_heads_q: int,
                          n_heads_kv: int, rope_base: float, softmax_scale: float | None = None,
                          out=None):
-    """A one-token step's attention in one launch: qkv (the QKV projection's
+    """A one-token step's attention in one launch (long caches of few
+    sequences: two, the second merging key splits): qkv (the QKV projection's
     K-split Partials, [B, 1, (Hq+2Hkv) D]) is split with RoPE at position
     *n_past (a one-element int32 device tensor), k / v are written to cache
     row *n_past, and q attends to rows 0 .. *n_past.  Returns o [B, Hq, D]."""
@@ -517,9 +523,13 @@ def decode_qkv_attention(qkv: "Partials", k_cache, v_cache, n_past, n_heads_q: i
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
     out = torch.empty((B, n_heads_q, D), dtype=k_cache.dtype, device=k_cache.device) \
         if out is None else out
-    call("teeny_decode_qkv_attention_dev", _p(qkv.slabs), qkv.n, _p(k_cache), _p(v_cache),
+    # few sequences over a long cache share each kv head's keys between workgroups
+    splits = decode_qkv_splits(B, n_heads_kv, L)
+    need = _lib.lib().teeny_decode_qkv_attention_workspace_bytes(B, n_heads_q, D, splits)
+    ws = torch.empty(need, dtype=torch.uint8, device=out.device) if need else None
+    call("teeny_decode_qkv_attention_split_dev", _p(qkv.slabs), qkv.n, _p(k_cache), _p(v_cache),
          _p(out), B, n_heads_q, n_heads_kv, D, L, _p(n_past), _ln(rope_base), scale,
-         _code(k_cache), _stream())
+         _code(k_cache), splits, _p(ws), need, _stream())
     return out
 
 

@@ -277,6 +277,8 @@ def test_decode_attention_f32_edges(cuda, B, Hq, Hkv, D, n_keys, L):
     (4, 32, 8, 128, 640),   # the Llama-3-8B decode shape
     (3, 8, 1, 64, 300),     # 8 q heads on one kv head, cache off the 32-key tile
     (2, 32, 1, 128, 1000),  # a 32-head group: every row of the score product
+    (1, 8, 2, 64, 1030),    # key splits: 5, the last ones without keys at small positions
+    (2, 32, 2, 128, 4200),  # 16 splits of one 32-key tile per wavefront and more
 ])
 def test_decode_qkv_attention_fused(cuda, B, Hq, Hkv, D, L):
     """The one-launch decode step (QKV split + RoPE + cache write +
