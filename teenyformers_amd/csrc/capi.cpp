@@ -873,17 +873,23 @@ static int norm_bwd_impl(bool ref_formula, const void* dy, const void* h, void* 
   if (!norm_shape(N, dtype, &vec, &ch)) return TEENY_ERR_UNSUPPORTED;
   if (!workspace || workspace_bytes < teeny_fused_add_rmsnorm_bwd_workspace_bytes(M, N))
     return TEENY_ERR_WORKSPACE;
-  int parts = norm_bwd_parts(M);
+  // workgroups of 16, 8 or 4 wavefronts (bwd_waves in norm.hip), a row each
+  // at a time; one dweight partial per workgroup
+  const int b = ch * vec * (int)dtype_size(dtype);
+  const int waves = b > 128 ? 4 : b > 64 || (vec == 1 && ch == 16) ? 8 : 16;
+  int parts = (M + waves - 1) / waves;
+  if (parts > kNormBwdMaxParts) parts = kNormBwdMaxParts;
   float* part = (float*)workspace;
   char name[64];
-  snprintf(name, sizeof name, "teeny_%s_bwd_%s_v%d_c%d", ref_formula ? "addnorm" : "rmsnorm",
-           dtype_tag(dtype), vec, ch);
+  snprintf(name, sizeof name, "teeny_%s_bwd_%s_v%d_c%d%s", ref_formula ? "addnorm" : "rmsnorm",
+           dtype_tag(dtype), vec, ch,
+           N == ch * 64 * vec && (dtype == TEENY_F32 || ch < 4) ? "_full" : "");
   void* a0[] = {&dy, &h, &dx, &dresidual, &part, &weight, &rstd, &M, &N};
-  int rc = launch(name, dim3(parts), dim3(256), 0, stream, a0);
+  int rc = launch(name, dim3(parts), dim3(64 * waves), 0, stream, a0);
   if (rc) return rc;
   snprintf(name, sizeof name, "teeny_rmsnorm_dw_reduce_%s", dtype_tag(dtype));
   void* a1[] = {&part, &dweight, &parts, &N};
-  return launch(name, dim3((N + 255) / 256), dim3(256), 0, stream, a1);
+  return launch(name, dim3((N + 31) / 32), dim3(1024), 0, stream, a1);
 }
 
 int teeny_fused_add_rmsnorm_bwd(const void* dy, const void* h, void* dx, void* dresidual,

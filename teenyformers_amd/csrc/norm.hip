@@ -149,98 +149,196 @@ __device__ __forceinline__ void rmsnorm_fwd_row(const T* __restrict__ x, const T
   }
 }
 
-// Rows are strided over a fixed number of workgroups; each wave keeps its
-// dweight partial in registers and the 4 waves combine through LDS.
-template <typename T, int VEC, int CH, bool REF>
-__device__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const T* __restrict__ h,
-                                 T* __restrict__ dx, T* __restrict__ dres,
-                                 float* __restrict__ dw_part, const T* __restrict__ w,
-                                 const float* __restrict__ rstd, int M, int N) {
-  __shared__ float red[kWaves - 1][CH * 64 * VEC];
+// A 16-byte vector (VEC > 1) or one element as loaded: rows wait in registers
+// in storage form, half the registers of fp32 values for bf16.
+template <typename T, int VEC>
+struct Raw {
+  T x;
+  DEVI void load(const T* p) { x = *p; }
+  DEVI float get(int) const { return (float)x; }
+  DEVI void hold() {}
+};
+template <>
+struct Raw<float, 4> {
+  f32x4 x;
+  DEVI void load(const float* p) { x = *reinterpret_cast<const f32x4*>(p); }
+  DEVI float get(int j) const { return x[j]; }
+  DEVI void hold() {}
+};
+template <>
+struct Raw<bf16, 8> {
+  u32x4 x;
+  DEVI void load(const bf16* p) { x = *reinterpret_cast<const u32x4*>(p); }
+  DEVI float get(int j) const { return j & 1 ? bf16hi(x[j / 2]) : bf16lo(x[j / 2]); }
+  // keeps the value packed up to here: widened once for two uses, it would
+  // hold twice the registers in between
+  DEVI void hold() { asm volatile("" : "+v"(x)); }
+};
+
+// Wavefronts per workgroup: the registers of a row (dy, h, w, the dweight
+// sums) allow 4, 2 or 1 wavefronts per SIMD, all in one workgroup per CU, so
+// that the dweight partials stay one per workgroup.
+template <typename T, int VEC, int CH>
+constexpr int bwd_waves() {
+  constexpr int B = CH * VEC * (int)sizeof(T);  // bytes of a row per lane
+  return B > 128 ? 4 : B > 64 || (VEC == 1 && CH == 16) ? 8 : 16;
+}
+
+// Rows are strided over the grid's wavefronts, which request their next row's
+// loads before they reduce and store the current one where the registers hold
+// it (PIPE: short rows, and fp32 rows, whose values need no widening); a
+// wavefront keeps its dweight sums in registers, and the workgroup adds them through LDS in a
+// fixed order (halves).  8192 rows of 2048 / 4096 / 8192 bf16, with the
+// reduction below: 25 / 44 / 100 us (4.0-4.6 TB/s), with one wavefront per
+// SIMD and fp32 rows in registers 94 / 158 / 414; fp32 8192 x 2048 40 us (117).
+template <typename T, int VEC, int CH, bool REF, bool FULL>
+__device__ __forceinline__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const T* __restrict__ h,
+                                                 T* __restrict__ dx, T* __restrict__ dres,
+                                                 float* __restrict__ dw_part,
+                                                 const T* __restrict__ w,
+                                                 const float* __restrict__ rstd, int M, int N) {
+  constexpr int NW = bwd_waves<T, VEC, CH>();
+  constexpr int B = CH * VEC * (int)sizeof(T);
+  constexpr bool PIPE = B <= 32 || (sizeof(T) == 4 && B >= 128);
+  __shared__ float red[NW / 2][CH * 64 * VEC];
   const int lane = threadIdx.x & 63;
   const int wave = threadIdx.x >> 6;
+  Raw<T, VEC> wr[CH];
   float dwacc[CH][VEC];
 #pragma unroll
-  for (int c = 0; c < CH; ++c)
+  for (int c = 0; c < CH; ++c) {
+    const int idx = (c * 64 + lane) * VEC;
+    if (FULL || idx < N) wr[c].load(w + idx);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) dwacc[c][j] = 0.0f;
+  }
   const float n_inv = 1.0f / (float)N;
-  for (int row = blockIdx.x * kWaves + wave; row < M; row += gridDim.x * kWaves) {
+  const int stride = gridDim.x * NW;
+  int row = blockIdx.x * NW + wave;
+  Raw<T, VEC> dyr[CH], hr[CH], dyn[PIPE ? CH : 1], hn[PIPE ? CH : 1];
+  float rs = 0.0f, rsn = 0.0f;
+  auto load = [&](int r, Raw<T, VEC>* a, Raw<T, VEC>* b, float& s) __attribute__((always_inline)) {
+    const long base = (long)r * N;
+    s = rstd[r];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int idx = (c * 64 + lane) * VEC;
+      if (FULL || idx < N) {
+        a[c].load(dy + base + idx);
+        b[c].load(h + base + idx);
+      }
+    }
+  };
+  if (row < M) load(row, dyr, hr, rs);
+  for (; row < M; row += stride) {
+    if constexpr (PIPE)
+      if (row + stride < M) load(row + stride, dyn, hn, rsn);
     const long base = (long)row * N;
-    const float rs = rstd[row];
-    float dyv[CH][VEC], hv[CH][VEC], wv[CH][VEC];
     float dot = 0.0f;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      int idx = (c * 64 + lane) * VEC;
-      if (idx < N) {
-        ldv<T, VEC>(dy + base + idx, dyv[c]);
-        ldv<T, VEC>(h + base + idx, hv[c]);
-        ldv<T, VEC>(w + idx, wv[c]);
+      const int idx = (c * 64 + lane) * VEC;
+      wr[c].hold();
+      if (FULL || idx < N)
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) dot += dyv[c][j] * wv[c][j] * hv[c][j];
-      }
+        for (int j = 0; j < VEC; ++j) dot += dyr[c].get(j) * wr[c].get(j) * hr[c].get(j);
     }
     dot = wave_sum(dot);
     const float rs2 = rs * rs;
     const float sc = dot * n_inv;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
-      int idx = (c * 64 + lane) * VEC;
-      if (idx < N) {
+      const int idx = (c * 64 + lane) * VEC;
+      dyr[c].hold();
+      hr[c].hold();
+      wr[c].hold();
+      if (FULL || idx < N) {
         float g[VEC];
 #pragma unroll
         for (int j = 0; j < VEC; ++j) {
-          g[j] = REF ? rs * wv[c][j] * (dyv[c][j] - hv[c][j] * rs2 * sc)
-                     : rs * (wv[c][j] * dyv[c][j] - hv[c][j] * rs2 * sc);
-          dwacc[c][j] += dyv[c][j] * hv[c][j] * rs;
+          const float dyv = dyr[c].get(j), hv = hr[c].get(j), wv = wr[c].get(j);
+          g[j] = REF ? rs * wv * (dyv - hv * rs2 * sc) : rs * (wv * dyv - hv * rs2 * sc);
+          dwacc[c][j] += dyv * hv * rs;
         }
         stv<T, VEC>(dx + base + idx, g);
         if (dres) stv<T, VEC>(dres + base + idx, g);
       }
     }
-  }
-  if (wave > 0) {
+    if constexpr (PIPE) {
 #pragma unroll
-    for (int c = 0; c < CH; ++c)
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) red[wave - 1][(c * 64 + lane) * VEC + j] = dwacc[c][j];
-  }
-  __syncthreads();
-  if (wave == 0) {
-#pragma unroll
-    for (int c = 0; c < CH; ++c) {
-      int idx = (c * 64 + lane) * VEC;
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) {
-        float s = dwacc[c][j];
-#pragma unroll
-        for (int wv2 = 0; wv2 < kWaves - 1; ++wv2) s += red[wv2][idx + j];
-        if (idx + j < N) dw_part[(long)blockIdx.x * N + idx + j] = s;
+      for (int c = 0; c < CH; ++c) {
+        dyr[c] = dyn[c];
+        hr[c] = hn[c];
       }
+      rs = rsn;
+    } else {
+      if (row + stride < M) load(row + stride, dyr, hr, rs);
     }
   }
+#pragma unroll
+  for (int s = NW / 2; s >= 1; s /= 2) {
+    if (wave >= s && wave < 2 * s)
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) red[wave - s][(c * VEC + j) * 64 + lane] = dwacc[c][j];
+    __syncthreads();
+    if (wave < s)
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+#pragma unroll
+        for (int j = 0; j < VEC; ++j) dwacc[c][j] += red[wave][(c * VEC + j) * 64 + lane];
+    __syncthreads();
+  }
+  if (wave == 0)
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+      const int idx = (c * 64 + lane) * VEC;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j)
+        if (idx + j < N) dw_part[(long)blockIdx.x * N + idx + j] = dwacc[c][j];
+    }
+}
+
+// dweight[n] += sum over workgroups of the partials (fixed order): 32 columns
+// per workgroup of 32 x 32 threads, thread (c, p) summing partials p, p + 32,
+// .. with 8 loads in flight, the 32 sums then added in order through LDS.
+// 256 partials of 2048: 4.7 us (a thread per column read them one after the
+// other on 8 workgroups: 61 us).
+template <typename T>
+__device__ void dw_reduce(const float* __restrict__ part, T* __restrict__ dw, int nparts, int N) {
+  __shared__ float red[32][33];
+  const int c = threadIdx.x & 31, p0 = threadIdx.x >> 5;
+  const int n = blockIdx.x * 32 + c;
+  float s = 0.0f;
+  if (n < N)
+    for (int p = p0; p < nparts; p += 32 * 8) {
+      float v[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)  // partials past the last re-read it and are not added
+        v[u] = part[(long)min(p + 32 * u, nparts - 1) * N + n];
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        if (p + 32 * u < nparts) s += v[u];
+    }
+  red[p0][c] = s;
+  __syncthreads();
+  if (p0 != 0 || n >= N) return;
+#pragma unroll
+  for (int p = 1; p < 32; ++p) s += red[p][c];
+  st(dw + n, ld(dw + n) + s);
 }
 
 }  // namespace
 
-// dweight[n] += sum over workgroups of the partials (fixed order).
-extern "C" __global__ __launch_bounds__(256) void teeny_rmsnorm_dw_reduce_f32(
+extern "C" __global__ __launch_bounds__(1024) void teeny_rmsnorm_dw_reduce_f32(
     const float* part, float* dw, int nparts, int N) {
-  int n = blockIdx.x * 256 + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.0f;
-  for (int p = 0; p < nparts; ++p) s += part[(long)p * N + n];
-  dw[n] = dw[n] + s;
+  dw_reduce(part, dw, nparts, N);
 }
 
-extern "C" __global__ __launch_bounds__(256) void teeny_rmsnorm_dw_reduce_bf16(
+extern "C" __global__ __launch_bounds__(1024) void teeny_rmsnorm_dw_reduce_bf16(
     const float* part, bf16* dw, int nparts, int N) {
-  int n = blockIdx.x * 256 + threadIdx.x;
-  if (n >= N) return;
-  float s = 0.0f;
-  for (int p = 0; p < nparts; ++p) s += part[(long)p * N + n];
-  dw[n] = (bf16)((float)dw[n] + s);
+  dw_reduce(part, dw, nparts, N);
 }
 
 // Few rows (a decode step's M = batch): one 256-thread workgroup per row, so
@@ -372,19 +470,23 @@ extern "C" __global__ __launch_bounds__(512) void teeny_addnorm_parts_fwd_bf16_v
                                                    float eps) {                                  \
     rmsnorm_fwd_row<T, VEC, CH, true, FULL>(x, res, y, h, rstd, w, M, N, eps);                   \
   }
-#define TEENY_NORM_INST(TN, T, VEC, CH)                                                          \
-  TEENY_NORM_FWD_INST(TN, T, VEC, CH, false, )                                                   \
-  TEENY_NORM_FWD_INST(TN, T, VEC, CH, true, _full)                                               \
-  extern "C" __global__ __launch_bounds__(256) void teeny_rmsnorm_bwd_##TN##_v##VEC##_c##CH(    \
-      const T* dy, const T* h, T* dx, T* dres, float* dw_part, const T* w, const float* rstd,    \
-      int M, int N) {                                                                            \
-    rmsnorm_bwd_rows<T, VEC, CH, false>(dy, h, dx, dres, dw_part, w, rstd, M, N);                \
+#define TEENY_NORM_BWD_INST(TN, T, VEC, CH, FULL, SFX)                                            \
+  extern "C" __global__ __launch_bounds__((64 * bwd_waves<T, VEC, CH>())) void                   \
+      teeny_rmsnorm_bwd_##TN##_v##VEC##_c##CH##SFX(const T* dy, const T* h, T* dx, T* dres,      \
+                                                   float* dw_part, const T* w,                   \
+                                                   const float* rstd, int M, int N) {            \
+    rmsnorm_bwd_rows<T, VEC, CH, false, FULL>(dy, h, dx, dres, dw_part, w, rstd, M, N);          \
   }                                                                                              \
-  extern "C" __global__ __launch_bounds__(256) void teeny_addnorm_bwd_##TN##_v##VEC##_c##CH(    \
-      const T* dy, const T* h, T* dx, T* dres, float* dw_part, const T* w, const float* rstd,    \
-      int M, int N) {                                                                            \
-    rmsnorm_bwd_rows<T, VEC, CH, true>(dy, h, dx, dres, dw_part, w, rstd, M, N);                 \
+  extern "C" __global__ __launch_bounds__((64 * bwd_waves<T, VEC, CH>())) void                   \
+      teeny_addnorm_bwd_##TN##_v##VEC##_c##CH##SFX(const T* dy, const T* h, T* dx, T* dres,      \
+                                                   float* dw_part, const T* w,                   \
+                                                   const float* rstd, int M, int N) {            \
+    rmsnorm_bwd_rows<T, VEC, CH, true, FULL>(dy, h, dx, dres, dw_part, w, rstd, M, N);           \
   }
+#define TEENY_NORM_INST(TN, T, VEC, CH)             \
+  TEENY_NORM_FWD_INST(TN, T, VEC, CH, false, )      \
+  TEENY_NORM_FWD_INST(TN, T, VEC, CH, true, _full)  \
+  TEENY_NORM_BWD_INST(TN, T, VEC, CH, false, )
 
 #define TEENY_NORM_ALL_CH(TN, T, VEC) \
   TEENY_NORM_INST(TN, T, VEC, 1)      \
@@ -397,3 +499,14 @@ TEENY_NORM_ALL_CH(f32, float, 4)
 TEENY_NORM_ALL_CH(f32, float, 1)
 TEENY_NORM_ALL_CH(bf16, bf16, 8)
 TEENY_NORM_ALL_CH(bf16, bf16, 1)
+
+// Backward rows of whole chunks without bounds tests; bf16 rows of 4 chunks or
+// more keep the tests (without them the compiler holds every chunk's widened
+// values at once and spills: 8192 x 2048 37 against 32 us).
+TEENY_NORM_BWD_INST(f32, float, 4, 1, true, _full)
+TEENY_NORM_BWD_INST(f32, float, 4, 2, true, _full)
+TEENY_NORM_BWD_INST(f32, float, 4, 4, true, _full)
+TEENY_NORM_BWD_INST(f32, float, 4, 8, true, _full)
+TEENY_NORM_BWD_INST(f32, float, 4, 16, true, _full)
+TEENY_NORM_BWD_INST(bf16, bf16, 8, 1, true, _full)
+TEENY_NORM_BWD_INST(bf16, bf16, 8, 2, true, _full)

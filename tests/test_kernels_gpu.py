@@ -198,6 +198,38 @@ def test_rmsnorm_bf16_bwd(cuda, m, n):
 # SwiGLU
 # ---------------------------------------------------------------------------
 
+@pytest.mark.parametrize("m,n,dtype", [
+    (m, n, t) for t in (torch.float32, torch.bfloat16)
+    for m, n in [(1, 8), (15, 33), (17, 520), (4099, 512), (8200, 40), (33, 1032), (300, 2048),
+                 (70, 4096), (9, 3000), (21, 1023)]] + [(5, 8192, torch.bfloat16)])
+def test_rmsnorm_bwd_edges(cuda, m, n, dtype):
+    """Backward at the edges of its workgroups (4, 8 or 16 rows), of the row
+    chunks and of the dweight reduction (32 columns, 1 to 256 partials), both
+    formulas, against float64 on the stored inputs.  fp32: sums of n (dx) and m
+    (dweight) terms, 2^-24 sqrt(terms) of the largest value; bf16: one rounding
+    more (2^-8 of each value)."""
+    g = torch.Generator(device="cuda").manual_seed(m * 31 + n)
+    dy, h = (torch.randn(m, n, generator=g, device="cuda").to(dtype) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(n, generator=g, device="cuda")).to(dtype)
+    rstd = (h.float().square().mean(-1) + 1e-5).rsqrt()
+    d, x, ww, r = dy.double(), h.double(), w.double(), rstd.double()[:, None]
+    dot = (d * ww * x).mean(-1, keepdim=True)
+    want = {"ref": r * ww * (d - x * r * r * dot), "true": r * (ww * d - x * r * r * dot)}
+    dw_want = (d * x * r).sum(0)
+    dx_ref, dres, dw_ref = ops.fused_add_rmsnorm_bwd(dy, h, w, rstd)
+    dx_true, dw_true = ops.rmsnorm_bwd(dy, h, w, rstd)
+    assert torch.equal(dx_ref, dres) and torch.equal(dw_ref, dw_true)
+    half = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+
+    def check(got, exact, terms):
+        tol = 4 * 2.0 ** -24 * max(4.0, terms) ** 0.5 * exact.abs().max() + half * exact.abs()
+        assert bool(((got.double() - exact).abs() <= tol).all())
+
+    check(dx_ref, want["ref"], n)
+    check(dx_true, want["true"], n)
+    check(dw_true, dw_want, m)
+
+
 def test_swiglu_reference_fixture(cuda):
     z = O.load_fixture("swiglu/input.bin").reshape(4, 16)
     got = host(ops.swiglu(dev(z)))
