@@ -388,12 +388,13 @@ DkdvPlan dkdv_plan(bool causal, int n_ctx_q, int n_ctx_k, int batch, int hq, int
 //   B2 Hq32 Hkv4 S264 D64 bidirectional     72 ->  42   (6)
 // and where the rule leaves one: B1 H32 S1024 D128 92 (103 with 2), B4 H4 S1090
 // 91 (95), B2 H8 S404 46 (50), B1 H32 S2048 207 (240), B1 Hq64 Hkv8 S8191 4312
-// (4415).
-int dkdv_share(int n_ctx_q, int n_ctx_k, int batch, int hq, int hkv) {
+// (4415), B4 Hq32 Hkv8 S200 D64 42 (44); two shares do not replace the two
+// wavefront groups (B2 Hq16 Hkv8 S2048 228, 238).
+int dkdv_share(int n_ctx_q, int n_ctx_k, int batch, int hq, int hkv, int head_dim) {
   const long cus = device_cus();
   const long wgs = (long)((n_ctx_k + 127) / 128) * batch * hkv;
   const long items = (long)(hq / hkv) * ((n_ctx_q + 31) / 32);
-  if (2 * wgs > cus && items < 96) return 1;
+  if ((2 * wgs > cus && items < 96) || items * head_dim < 2560) return 1;
   const long s2 = std::min(2 * cus / wgs, items / 12);
   const long s4 = wgs <= cus ? std::min(4 * cus / wgs, items / 64) : 1;
   const long s = std::min(std::max(s2, s4), 16L);
@@ -459,8 +460,8 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
     DkdvPlan plan = dkdv_plan(causal, n_ctx_q, n_ctx_k, batch, hq, hkv, dtype);
     const size_t base = fa2_bwd_ws(n_ctx_q, batch, hq, head_dim, dtype);
     if (plan.split == 1) {
-      const int share = dkdv_share(n_ctx_q, n_ctx_k, batch, hq, hkv);
-      if (share > 1 &&
+      const int share = dkdv_share(n_ctx_q, n_ctx_k, batch, hq, hkv, head_dim);
+      if (share > plan.groups &&
           workspace_bytes >= base + dkdv_split_bytes(n_ctx_k, batch, hkv, head_dim, share))
         plan = DkdvPlan{1, share};
     }
@@ -729,7 +730,7 @@ size_t teeny_flash_attn2_bwd_workspace_bytes_shared(int n_ctx_q, int n_ctx_k, in
   dtype &= ~TEENY_GRAD_F32;
   const int share = dtype == TEENY_F32
                         ? dkdv_f32_split(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv)
-                        : dkdv_share(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv);
+                        : dkdv_share(n_ctx_q, n_ctx_k, batch, n_heads_q, n_heads_kv, head_dim);
   const size_t shared = fa2_bwd_ws(n_ctx_q, batch, n_heads_q, head_dim, dtype) +
                         dkdv_split_bytes(n_ctx_k, batch, n_heads_kv, head_dim, share);
   return shared > gqa ? shared : gqa;

@@ -426,8 +426,8 @@ def test_fa2_bf16_bwd_gqa_split(cuda, grad_f32):
 @pytest.mark.parametrize("grad_f32", [False, True])
 @pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
     (1, 8, 2, 421, 421, 128, True),    # GQA: shares of 56 items cross head boundaries
-    (1, 2, 2, 800, 130, 64, False),    # MHA, bidirectional, two key blocks
-    (1, 8, 1, 97, 300, 64, True),      # causal blocks past the last query row: empty shares
+    (1, 2, 2, 2000, 130, 64, False),    # MHA, bidirectional, two key blocks
+    (1, 8, 1, 200, 300, 64, True),     # causal blocks past the last query row: empty shares
     (1, 4, 1, 2050, 2050, 64, True),   # instead of the two-group kernel, 16 shares
 ])
 def test_fa2_bf16_bwd_shared_walk(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32):
