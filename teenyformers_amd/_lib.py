@@ -29,6 +29,7 @@ class TeenyError(RuntimeError):
 
 
 _lib = None
+_fns: dict = {}  # entry points by name, for call()
 
 _p = ctypes.c_void_p
 _i = ctypes.c_int
@@ -131,7 +132,12 @@ def check(rc: int, what: str) -> None:
 
 def call(name: str, *args) -> None:
     """Call a status-returning entry point and raise on a nonzero status."""
-    check(getattr(lib(), name)(*args), name)
+    fn = _fns.get(name)
+    if fn is None:
+        fn = _fns[name] = getattr(lib(), name)
+    rc = fn(*args)
+    if rc != 0:
+        check(rc, name)
 
 
 def profile_enable(on: bool) -> None:

@@ -34,12 +34,20 @@ MI355X-specific structure (same arithmetic):
 from __future__ import annotations
 
 import dataclasses
+import functools
 import json
 import math
 
 import torch
 
 from . import ops
+
+
+@functools.lru_cache(maxsize=64)
+def _f32_rsqrt(n: int) -> float:
+    """1 / sqrt(n) in fp32 arithmetic (asked once per attention call)."""
+    return float(torch.tensor(1.0, dtype=torch.float32)
+                 / torch.tensor(float(n), dtype=torch.float32).sqrt())
 
 
 @dataclasses.dataclass
@@ -65,8 +73,7 @@ class LlamaConfig:
         return -(-raw // 64) * 64
 
     def softmax_scale(self) -> float:  # config.rs:156-158 (f32)
-        return float(torch.tensor(1.0, dtype=torch.float32)
-                     / torch.tensor(float(self.head_dim()), dtype=torch.float32).sqrt())
+        return _f32_rsqrt(self.head_dim())
 
     def n_kv_heads(self) -> int:  # config.rs:161-163
         return self.n_kv_heads_ if self.n_kv_heads_ is not None else self.n_heads
@@ -162,12 +169,16 @@ def load_hf_weights(cfg: LlamaConfig, model_dir: str, dtype=torch.bfloat16,
 
 class KVCache:
     """Per-layer K/V caches [B, Hkv, capacity, D], zero-initialised (rows past
-    the written prefix are masked by causality and must hold finite values)."""
+    the written prefix are masked by causality and must hold finite values).
+    prompt_only: the prompt writes every row before any is read, so none is
+    initialised."""
 
-    def __init__(self, cfg: LlamaConfig, batch: int, capacity: int, dtype, device="cuda"):
+    def __init__(self, cfg: LlamaConfig, batch: int, capacity: int, dtype, device="cuda",
+                 prompt_only: bool = False):
         shape = (batch, cfg.n_kv_heads(), capacity, cfg.head_dim())
-        self.k = [torch.zeros(shape, dtype=dtype, device=device) for _ in range(cfg.n_layers)]
-        self.v = [torch.zeros(shape, dtype=dtype, device=device) for _ in range(cfg.n_layers)]
+        new = torch.empty if prompt_only else torch.zeros
+        self.k = [new(shape, dtype=dtype, device=device) for _ in range(cfg.n_layers)]
+        self.v = [new(shape, dtype=dtype, device=device) for _ in range(cfg.n_layers)]
         self.capacity = capacity
         self.length = 0
 
@@ -338,7 +349,8 @@ class Llama:
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         """All-position logits [B, S, vocab] (src/llama.rs:65-81)."""
         B, S = ids.shape
-        cache = KVCache(self.cfg, B, S, self.w["model.norm.weight"].dtype, ids.device)
+        cache = KVCache(self.cfg, B, S, self.w["model.norm.weight"].dtype, ids.device,
+                        prompt_only=True)
         return self.logits(self.hidden(ids, cache, 0))
 
     # -- generation -----------------------------------------------------------
@@ -388,7 +400,8 @@ class Llama:
         out = []
         for _ in range(n_new):
             B, S = seq.shape
-            cache = KVCache(self.cfg, B, S, self.w["model.norm.weight"].dtype, seq.device)
+            cache = KVCache(self.cfg, B, S, self.w["model.norm.weight"].dtype, seq.device,
+                            prompt_only=True)
             h = self.hidden(seq, cache, 0)
             nxt = ops.argmax_rows(self.logits(h[:, -1])).view(-1, 1)
             out.append(nxt)
@@ -400,7 +413,8 @@ def block_forward(cfg: LlamaConfig, w: dict, x: torch.Tensor, layer: int = 0) ->
     """One LlamaBlock forward, x [B, S, d] -> [B, S, d] (src/layers/llama_block.rs:55-65)."""
     model = Llama(cfg, w)
     B, S, d = x.shape
-    cache = KVCache(dataclasses.replace(cfg, n_layers=layer + 1), B, S, x.dtype, x.device)
+    cache = KVCache(dataclasses.replace(cfg, n_layers=layer + 1), B, S, x.dtype, x.device,
+                    prompt_only=True)
     p = f"model.layers.{layer}."
     n1, _ = ops.rmsnorm(x, w[p + "input_layernorm.weight"], cfg.eps, want_rstd=False)
     a = model._attention(layer, n1, cache, 0)
