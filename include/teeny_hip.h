@@ -281,6 +281,13 @@ int teeny_rmsnorm_fwd(const void* x, void* y, float* rstd, const void* weight, i
 int teeny_rmsnorm_bwd(const void* dy, const void* x, void* dx, void* dweight, const void* weight,
                       const float* rstd, int M, int N, int dtype, void* workspace,
                       size_t workspace_bytes, hipStream_t stream);
+/* teeny_fused_add_rmsnorm_bwd (fused 1) or teeny_rmsnorm_bwd (fused 0,
+ * dresidual null) with dweight written instead of accumulated into: a fresh
+ * dweight needs no zeros. */
+int teeny_rmsnorm_bwd_set(int fused, const void* dy, const void* h, void* dx, void* dresidual,
+                          void* dweight, const void* weight, const float* rstd, int M, int N,
+                          int dtype, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream);
 
 /* --------------------------------------------------------------------------
  * SwiGLU: z [M, 2*d_ff] (gate || up) -> out [M, d_ff].

@@ -66,6 +66,7 @@ _SIGNATURES = {
     "teeny_fused_add_rmsnorm_bwd_workspace_bytes": ([_i, _i], _sz),
     "teeny_rmsnorm_fwd": ([_p] * 4 + [_i, _i, _f, _i, _p], _i),
     "teeny_rmsnorm_bwd": ([_p] * 6 + [_i, _i, _i, _p, _sz, _p], _i),
+    "teeny_rmsnorm_bwd_set": ([_i] + [_p] * 7 + [_i, _i, _i, _p, _sz, _p], _i),
     "teeny_swiglu_fwd": ([_p, _p, _i, _i, _i, _p], _i),
     "teeny_swiglu_bwd": ([_p, _p, _p, _i, _i, _i, _p], _i),
     "teeny_add": ([_p, _p, _p, ctypes.c_long, _i, _p], _i),

@@ -866,7 +866,7 @@ size_t teeny_fused_add_rmsnorm_bwd_workspace_bytes(int M, int N) {
 static int norm_bwd_impl(bool ref_formula, const void* dy, const void* h, void* dx,
                          void* dresidual, void* dweight, const void* weight, const float* rstd,
                          int M, int N, int dtype, void* workspace, size_t workspace_bytes,
-                         hipStream_t stream) {
+                         hipStream_t stream, int add_dw = 1) {
   if (!dy || !h || !dx || !dweight || !weight || !rstd) return TEENY_ERR_NULL_POINTER;
   if (!dtype_ok(dtype)) return TEENY_ERR_UNSUPPORTED;
   if (M <= 0 || N <= 0 || (long)M * N >= kMaxElems) return TEENY_ERR_INVALID_SHAPE;
@@ -889,7 +889,7 @@ static int norm_bwd_impl(bool ref_formula, const void* dy, const void* h, void* 
   int rc = launch(name, dim3(parts), dim3(64 * waves), 0, stream, a0);
   if (rc) return rc;
   snprintf(name, sizeof name, "teeny_rmsnorm_dw_reduce_%s", dtype_tag(dtype));
-  void* a1[] = {&part, &dweight, &parts, &N};
+  void* a1[] = {&part, &dweight, &parts, &N, &add_dw};
   return launch(name, dim3((N + 31) / 32), dim3(1024), 0, stream, a1);
 }
 
@@ -906,6 +906,15 @@ int teeny_rmsnorm_bwd(const void* dy, const void* x, void* dx, void* dweight, co
                       size_t workspace_bytes, hipStream_t stream) {
   return norm_bwd_impl(false, dy, x, dx, nullptr, dweight, weight, rstd, M, N, dtype, workspace,
                        workspace_bytes, stream);
+}
+
+int teeny_rmsnorm_bwd_set(int fused, const void* dy, const void* h, void* dx, void* dresidual,
+                          void* dweight, const void* weight, const float* rstd, int M, int N,
+                          int dtype, void* workspace, size_t workspace_bytes,
+                          hipStream_t stream) {
+  if (fused < 0 || fused > 1 || (!fused && dresidual)) return TEENY_ERR_INVALID_VALUE;
+  return norm_bwd_impl(fused != 0, dy, h, dx, dresidual, dweight, weight, rstd, M, N, dtype,
+                       workspace, workspace_bytes, stream, 0);
 }
 
 static int swiglu_impl(bool bwd, const void* grad, const void* z, void* out, int M, int d_ff,

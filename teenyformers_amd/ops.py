@@ -365,9 +365,14 @@ def fused_add_rmsnorm_bwd(dy, h, weight, rstd, dweight=None, want_dres: bool = T
     M, N = _rows(dy)
     dx = torch.empty_like(dy)
     dres = torch.empty_like(dy) if want_dres else None
+    ws = _norm_ws(M, N, dy.device)
+    if dweight is None and weight.numel() == N:  # written whole: no zeros first
+        dweight = torch.empty_like(weight)
+        call("teeny_rmsnorm_bwd_set", 1, _p(dy), _p(h), _p(dx), _p(dres), _p(dweight),
+             _p(weight), _p(rstd), M, N, _code(dy), _p(ws), ws.numel(), _stream())
+        return dx, dres, dweight
     if dweight is None:
         dweight = torch.zeros_like(weight)
-    ws = _norm_ws(M, N, dy.device)
     call("teeny_fused_add_rmsnorm_bwd", _p(dy), _p(h), _p(dx), _p(dres), _p(dweight), _p(weight),
          _p(rstd), M, N, _code(dy), _p(ws), ws.numel(), _stream())
     return dx, dres, dweight
@@ -378,9 +383,14 @@ def rmsnorm_bwd(dy, x, weight, rstd, dweight=None):
     _dev(dy, x, weight, rstd)
     M, N = _rows(dy)
     dx = torch.empty_like(dy)
+    ws = _norm_ws(M, N, dy.device)
+    if dweight is None and weight.numel() == N:  # written whole: no zeros first
+        dweight = torch.empty_like(weight)
+        call("teeny_rmsnorm_bwd_set", 0, _p(dy), _p(x), _p(dx), 0, _p(dweight), _p(weight),
+             _p(rstd), M, N, _code(dy), _p(ws), ws.numel(), _stream())
+        return dx, dweight
     if dweight is None:
         dweight = torch.zeros_like(weight)
-    ws = _norm_ws(M, N, dy.device)
     call("teeny_rmsnorm_bwd", _p(dy), _p(x), _p(dx), _p(dweight), _p(weight), _p(rstd), M, N,
          _code(dy), _p(ws), ws.numel(), _stream())
     return dx, dweight

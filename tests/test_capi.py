@@ -183,6 +183,8 @@ def test_other_ops_validation(L):
     assert L.teeny_rmsnorm_fwd(P, P, None, P, 4, 64 * 8 * 32, 1e-5, BF16, None) == UNSUP
     assert L.teeny_fused_add_rmsnorm_fwd(P, P, P, P, None, P, 4, 16, 1e-6, F32, None) == NULLP
     assert L.teeny_fused_add_rmsnorm_bwd(P, P, P, P, P, P, P, 4, 16, F32, None, 0, None) == WS
+    assert L.teeny_rmsnorm_bwd_set(0, P, P, P, P, P, P, P, 4, 16, F32, P, 1 << 20, None) == VALUE
+    assert L.teeny_rmsnorm_bwd_set(1, P, P, P, P, P, P, P, 4, 16, F32, None, 0, None) == WS
     assert L.teeny_swiglu_fwd(P, P, 0, 8, F32, None) == SHAPE
     assert L.teeny_token_embed_fwd(P, P, P, 4, 16, 10, BF16, F32, None) == UNSUP  # ids dtype
 

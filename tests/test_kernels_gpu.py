@@ -219,6 +219,10 @@ def test_rmsnorm_bwd_edges(cuda, m, n, dtype):
     dx_ref, dres, dw_ref = ops.fused_add_rmsnorm_bwd(dy, h, w, rstd)
     dx_true, dw_true = ops.rmsnorm_bwd(dy, h, w, rstd)
     assert torch.equal(dx_ref, dres) and torch.equal(dw_ref, dw_true)
+    # a dweight written whole is the one accumulated into zeros
+    zeros = lambda: torch.zeros_like(w)  # noqa: E731
+    assert torch.equal(ops.rmsnorm_bwd(dy, h, w, rstd, zeros())[1], dw_true)
+    assert torch.equal(ops.fused_add_rmsnorm_bwd(dy, h, w, rstd, zeros())[2], dw_ref)
     half = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
 
     def check(got, exact, terms):
