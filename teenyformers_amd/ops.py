@@ -460,8 +460,14 @@ def token_embed(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
 # ---------------------------------------------------------------------------
 
 @functools.lru_cache(maxsize=64)
-def _ln(rope_base: float) -> float:
+def _ln_f32(rope_base: float) -> float:
     return float(torch.tensor(rope_base, dtype=torch.float32).log().item())
+
+
+def _ln(rope_base) -> float:
+    """ln of the RoPE base in fp32, kept by the base's value (a tensor would be
+    a key by its identity)."""
+    return _ln_f32(float(rope_base))
 
 
 def qkv_rope_split(qkv, q_out, k_cache, v_cache, pos0, n_heads_q: int, n_heads_kv: int,

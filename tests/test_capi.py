@@ -342,3 +342,14 @@ def test_header_is_c(tmp_path):
                     str(src), "-L" + libdir, "-lteeny_hip", "-Wl,-rpath," + libdir,
                     "-o", str(exe)], check=True)
     assert subprocess.run([str(exe)]).returncode == 0
+
+
+def test_rope_base_tensor_by_value():
+    """The kept ln(base) follows the value of a base given as a tensor."""
+    import torch
+
+    from teenyformers_amd import ops
+    base = torch.tensor(1e4)
+    first = ops._ln(base)
+    base.fill_(5e5)
+    assert first == ops._ln(1e4) and ops._ln(base) == ops._ln(5e5) != first
