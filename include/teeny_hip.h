@@ -42,7 +42,7 @@ extern "C" {
 
 #define TEENY_ABI_VERSION 1
 
-typedef enum { TEENY_F32 = 0, TEENY_BF16 = 1, TEENY_I32 = 2 } teeny_dtype;
+typedef enum { TEENY_F32 = 0, TEENY_BF16 = 1, TEENY_I32 = 2, TEENY_I64 = 3 } teeny_dtype;
 
 /* Or-ed into the dtype of a flash-attention backward (and its workspace
  * queries): with TEENY_BF16 inputs, dq, dk and dv are fp32 gradients, as the
@@ -314,6 +314,12 @@ int teeny_add(const void* a, const void* b, void* y, long n, int dtype, hipStrea
 int teeny_token_embed_fwd(const void* ids, const void* weight, void* out, int seq_len,
                           int d_model, int vocab_size, int ids_dtype, int dtype,
                           hipStream_t stream);
+/* The gather and the first block's RMSNorm in one launch, for up to 255 rows:
+ * h[s, :] = table[ids[s], :], y = rmsnorm(h) * weight; ids_dtype TEENY_I32 or
+ * TEENY_I64.  The bits of teeny_token_embed_fwd, then teeny_rmsnorm_fwd. */
+int teeny_embed_rmsnorm_fwd(const void* ids, const void* table, void* h, void* y,
+                            const void* weight, int M, int N, int vocab, float eps,
+                            int ids_dtype, int dtype, hipStream_t stream);
 
 /* --------------------------------------------------------------------------
  * Llama attention plumbing (extensions; no single reference op).
@@ -369,6 +375,10 @@ int teeny_decode_attention_dev(const void* q, const void* k_cache, const void* v
  * panics, counts as the maximum (the last NaN wins). */
 int teeny_argmax_rows(const void* x, int64_t* out, int rows, int cols, int dtype,
                       hipStream_t stream);
+/* ... and, if advance is not null, *advance += 1 (int32, device): a captured
+ * decode step's position moves on with the token that it chose. */
+int teeny_argmax_rows_advance(const void* x, int64_t* out, int rows, int cols, int dtype,
+                              int* advance, hipStream_t stream);
 
 /* Linear layer y[M, N] = x[M, K] . w[N, K]^T in bf16, any M >= 1: replaces
  * the external teeny-core Linear behind sym_linear (src/layers/mod.rs:54-58).

@@ -13,7 +13,7 @@ PKG = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(PKG, "libteeny_hip.so")
 HEADER = os.path.join(os.path.dirname(PKG), "include", "teeny_hip.h")
 
-TEENY_F32, TEENY_BF16, TEENY_I32 = 0, 1, 2
+TEENY_F32, TEENY_BF16, TEENY_I32, TEENY_I64 = 0, 1, 2, 3
 TEENY_LINEAR_PLAIN, TEENY_LINEAR_SWIGLU, TEENY_LINEAR_PARTIALS = 0, 1, 2
 TEENY_GRAD_F32 = 0x100  # or-ed into a bf16 backward's dtype: fp32 dq/dk/dv
 
@@ -83,6 +83,8 @@ _SIGNATURES = {
     "teeny_decode_qkv_attention_workspace_bytes": ([_i] * 4, _sz),
     "teeny_decode_qkv_attention_split_dev": ([_p, _i, _p, _p, _p] + [_i] * 5 + [_p, _f, _f, _i, _i,
                                                                              _p, _sz, _p], _i),
+    "teeny_embed_rmsnorm_fwd": ([_p] * 5 + [_i, _i, _i, _f, _i, _i, _p], _i),
+    "teeny_argmax_rows_advance": ([_p, _p, _i, _i, _i, _p, _p], _i),
     "teeny_argmax_rows": ([_p, _p, _i, _i, _i, _p], _i),
     "teeny_linear_bf16": ([_p, _p, _p, _i, _i, _i, _p], _i),
     "teeny_gemm_bf16": ([_p, _p, _p, _i, _i, _i, _p], _i),

@@ -846,6 +846,28 @@ int teeny_fused_add_rmsnorm_partials_fwd(const float* parts, int n_parts, const 
   return launch(name, dim3(M), dim3(256), 0, stream, args);
 }
 
+// The rows that norm_fwd_impl gives a workgroup each, with its kernels' shapes
+// and the same bits as teeny_token_embed_fwd followed by teeny_rmsnorm_fwd.
+int teeny_embed_rmsnorm_fwd(const void* ids, const void* table, void* h, void* y,
+                            const void* weight, int M, int N, int vocab, float eps,
+                            int ids_dtype, int dtype, hipStream_t stream) {
+  if (!ids || !table || !h || !y || !weight) return TEENY_ERR_NULL_POINTER;
+  if (!dtype_ok(dtype) || (ids_dtype != TEENY_I64 && ids_dtype != TEENY_I32))
+    return TEENY_ERR_UNSUPPORTED;
+  if (M <= 0 || N <= 0 || vocab <= 0 || (long)vocab * N >= kMaxElems * 2)
+    return TEENY_ERR_INVALID_SHAPE;
+  if (!(eps >= 0.0f) || !std::isfinite(eps)) return TEENY_ERR_INVALID_VALUE;
+  int vec, ch;
+  if (M >= 256 || !norm_shape(N, dtype, &vec, &ch) || vec == 1) return TEENY_ERR_UNSUPPORTED;
+  const bool t512 = dtype == TEENY_BF16 && ch == 8;
+  char name[64];
+  snprintf(name, sizeof name, "teeny_embed_rmsnorm_%s_%s_c%d%s", dtype_tag(dtype),
+           ids_dtype == TEENY_I32 ? "i32" : "i64", t512 || ch <= 4 ? 1 : ch / 4,
+           t512 ? "_t512" : "");
+  void* args[] = {&ids, &table, &h, &y, &weight, &N, &vocab, &eps};
+  return launch(name, dim3(M), dim3(t512 ? 512 : 256), 0, stream, args);
+}
+
 int teeny_fused_add_rmsnorm_fwd(const void* x, const void* residual, void* y, void* h,
                                 float* rstd, const void* weight, int M, int N, float eps,
                                 int dtype, hipStream_t stream) {
@@ -1221,13 +1243,18 @@ int teeny_decode_attention_dev(const void* q, const void* k_cache, const void* v
 
 int teeny_argmax_rows(const void* x, int64_t* out, int rows, int cols, int dtype,
                       hipStream_t stream) {
+  return teeny_argmax_rows_advance(x, out, rows, cols, dtype, nullptr, stream);
+}
+
+int teeny_argmax_rows_advance(const void* x, int64_t* out, int rows, int cols, int dtype,
+                              int* advance, hipStream_t stream) {
   if (!x || !out) return TEENY_ERR_NULL_POINTER;
   if (!dtype_ok(dtype)) return TEENY_ERR_UNSUPPORTED;
   if (rows <= 0 || cols <= 0 || (long)rows * cols >= kMaxElems * 2)
     return TEENY_ERR_INVALID_SHAPE;
   char name[48];
   snprintf(name, sizeof name, "teeny_argmax_rows_%s", dtype_tag(dtype));
-  void* args[] = {&x, &out, &cols};
+  void* args[] = {&x, &out, &cols, &advance};
   return launch(name, dim3(rows), dim3(1024), 0, stream, args);
 }
 

@@ -464,12 +464,16 @@ __device__ void decode_combine(const float* __restrict__ pm, const float* __rest
 // Row argmax: one workgroup of 1024 threads per row, 16-byte loads; the
 // last index of the maximum, as the reference's greedy_sample
 // (examples/llama_generate.rs:252-257, Iterator::max_by); NaN, on which the
-// reference's comparison panics, counts as the maximum.
+// reference's comparison panics, counts as the maximum.  advance, if given, is
+// a counter that goes up by one (a captured step's position, which every
+// earlier kernel of the stream has read; a launch of its own took 3.9 us).
 constexpr int kArgThreads = 1024;
 template <typename T>
-__device__ void argmax_rows(const T* __restrict__ x, long long* __restrict__ out, int cols) {
+__device__ void argmax_rows(const T* __restrict__ x, long long* __restrict__ out, int cols,
+                            int* __restrict__ advance) {
   __shared__ float bv[kArgThreads / 64];
   __shared__ int bi[kArgThreads / 64];
+  if (advance && blockIdx.x == 0 && threadIdx.x == 0) *advance += 1;
   const T* row = x + (long)blockIdx.x * cols;
   float v = -INFINITY;
   int idx = -1;
@@ -598,8 +602,8 @@ TEENY_QKV_PARTS_INST(bf16, bf16)
     decode_combine<T>(pm, pl, po, o, n_chunks, head_dim);                                       \
   }                                                                                             \
   extern "C" __global__ __launch_bounds__(1024) void teeny_argmax_rows_##TN(                   \
-      const T* x, long long* out, int cols) {                                                   \
-    argmax_rows<T>(x, out, cols);                                                               \
+      const T* x, long long* out, int cols, int* advance) {                                     \
+    argmax_rows<T>(x, out, cols, advance);                                                      \
   }
 
 // bf16 caches that the matrix-core kernel (decode_bf16.hip) does not take

@@ -317,8 +317,9 @@ class Llama:
         after the attention add, and the FFN output (the block's output is
         the sum of the last two)."""
         cfg, w = self.cfg, self.w
-        x = ops.token_embed(ids.to(torch.int32).contiguous(), w["model.embed_tokens.weight"])
         eps = cfg.eps
+        x, n1 = ops.embed_rmsnorm(ids, w["model.embed_tokens.weight"],
+                                  w["model.layers.0.input_layernorm.weight"], eps)
         pos = pos0
         if ids.shape[1] == 1 and not isinstance(pos0, torch.Tensor) and pos0 > 0:
             # a one-token step takes its position from device memory, as the
@@ -327,9 +328,7 @@ class Llama:
         delta = None
         for i in range(cfg.n_layers):
             p = f"model.layers.{i}."
-            if delta is None:
-                n1, _ = ops.rmsnorm(x, w[p + "input_layernorm.weight"], eps, want_rstd=False)
-            else:  # x = x + ffn(...) fused into this block's input norm
+            if i > 0:  # x = x + ffn(...) fused into this block's input norm
                 n1, x, _ = ops.fused_add_rmsnorm(delta, x, w[p + "input_layernorm.weight"], eps)
             x_in = x
             a = self._attention(i, n1, cache, pos)
@@ -476,8 +475,8 @@ class DecodeGraph:
             self.logits = m.logits(h[:, -1])
             # the greedy choice lands in the ids the next replay embeds (the
             # embedding read them at the start of this step)
-            ops.argmax_rows(self.logits, out=self.ids.view(-1))
-        self.pos.add_(1)
+            # (and the position moves on: every kernel that reads it came before)
+            ops.argmax_rows(self.logits, out=self.ids.view(-1), advance=self.pos)
 
     def replay(self):
         if self.cache.length >= self.cache.capacity:

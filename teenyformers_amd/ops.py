@@ -16,7 +16,7 @@ import threading
 import torch
 
 from . import _lib
-from ._lib import TEENY_BF16, TEENY_F32, TEENY_I32, call
+from ._lib import TEENY_BF16, TEENY_F32, TEENY_I32, TEENY_I64, call
 
 _DTYPES = {torch.float32: TEENY_F32, torch.bfloat16: TEENY_BF16}
 
@@ -455,6 +455,25 @@ def token_embed(ids: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
     return out
 
 
+def embed_rmsnorm(ids: torch.Tensor, weight: torch.Tensor, norm_weight: torch.Tensor, eps: float):
+    """token_embed and the first block's rmsnorm -> (x, y) [..., d_model], for integer ids.
+    Few rows of whole 16-byte vectors (a decode step, a short prompt) take one launch."""
+    V, Dm = weight.shape
+    vn = 8 if weight.dtype == torch.bfloat16 else 4
+    if (not 0 < ids.numel() < 256 or Dm % vn != 0 or Dm > 1024 * vn
+            or ids.dtype not in (torch.int32, torch.int64) or norm_weight.dtype != weight.dtype):
+        x = token_embed(ids.to(torch.int32).contiguous(), weight)
+        return x, rmsnorm(x, norm_weight, eps, want_rstd=False)[0]
+    ids = ids.contiguous()
+    _dev(ids, weight, norm_weight)
+    x = torch.empty(ids.shape + (Dm,), dtype=weight.dtype, device=weight.device)
+    y = torch.empty_like(x)
+    call("teeny_embed_rmsnorm_fwd", _p(ids), _p(weight), _p(x), _p(y), _p(norm_weight),
+         ids.numel(), Dm, V, float(eps), TEENY_I32 if ids.dtype == torch.int32 else TEENY_I64,
+         _code(weight), _stream())
+    return x, y
+
+
 # ---------------------------------------------------------------------------
 # Llama attention plumbing
 # ---------------------------------------------------------------------------
@@ -562,17 +581,21 @@ def decode_qkv_attention(qkv: "Partials", k_cache, v_cache, n_past, n_heads_q: i
     return out
 
 
-def argmax_rows(x, out=None):
+def argmax_rows(x, out=None, advance=None):
     """x [rows, cols] -> int64 [rows]: the last index of each row's maximum,
     the reference's greedy choice (examples/llama_generate.rs:252-257,
-    Iterator::max_by); NaN counts as the maximum."""
+    Iterator::max_by); NaN counts as the maximum.  advance: an int32 device
+    counter that goes up by one."""
     _dev(x)
     x2 = x.reshape(-1, x.shape[-1])
     if not x2.is_contiguous():
         x2 = x2.contiguous()
     rows, cols = x2.shape
     out = torch.empty(rows, dtype=torch.int64, device=x.device) if out is None else out
-    call("teeny_argmax_rows", _p(x2), _p(out), rows, cols, _code(x2), _stream())
+    if advance is not None:
+        _dev(advance)
+    call("teeny_argmax_rows_advance", _p(x2), _p(out), rows, cols, _code(x2), _p(advance),
+         _stream())
     return out
 
 

@@ -227,6 +227,11 @@ def test_decode_ops_validation(L):
                                                9.21, BF16, None) == SHAPE  # 8 % 3
     assert L.teeny_argmax_rows(None, P, 4, 10, BF16, None) == NULLP
     assert L.teeny_argmax_rows(P, P, 0, 10, BF16, None) == SHAPE
+    assert L.teeny_argmax_rows_advance(None, P, 4, 10, BF16, P, None) == NULLP
+    assert L.teeny_embed_rmsnorm_fwd(P, P, P, P, P, 256, 64, 10, 1e-5, 3, BF16, None) == UNSUP
+    assert L.teeny_embed_rmsnorm_fwd(P, P, P, P, P, 4, 60, 10, 1e-5, 3, BF16, None) == UNSUP
+    assert L.teeny_embed_rmsnorm_fwd(P, P, P, P, P, 4, 64, 10, 1e-5, F32, BF16, None) == UNSUP
+    assert L.teeny_embed_rmsnorm_fwd(P, P, P, P, None, 4, 64, 10, 1e-5, 3, BF16, None) == NULLP
 
 
 def test_decode_qkv_attention_validation(L):

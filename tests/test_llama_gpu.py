@@ -225,6 +225,26 @@ def test_argmax_rows(cuda, dtype):
     # a row whose length is not a multiple of the vector width
     y = x[:, :1001].contiguous()
     assert torch.equal(ops.argmax_rows(y), 1000 - torch.argmax(y.flip(-1), dim=-1))
+    pos = torch.tensor([41, 7], dtype=torch.int32, device="cuda")
+    assert torch.equal(ops.argmax_rows(x, advance=pos[:1]), got) and pos.tolist() == [42, 7]
+
+
+@pytest.mark.parametrize("rows,N,dtype", [
+    (r, n, t) for t in (torch.float32, torch.bfloat16)
+    for r, n in [(1, 8), (3, 520), (255, 1024), (256, 64), (16, 2048), (5, 4096), (2, 1002)]]
+    + [(2, 8192, torch.bfloat16), (3, 1028, torch.float32)])
+@pytest.mark.parametrize("idt", [torch.int64, torch.int32])
+def test_embed_rmsnorm(cuda, rows, N, dtype, idt):
+    """The gather and the first norm in one launch (and the shapes that keep
+    two) have the bits of token_embed, then rmsnorm; ids outside the table too."""
+    g = torch.Generator(device="cuda").manual_seed(rows + N)
+    table = torch.randn(37, N, generator=g, device="cuda").to(dtype)
+    w = torch.randn(N, generator=g, device="cuda").to(dtype)
+    ids = torch.randint(-1, 38, (rows, 1), generator=g, device="cuda").to(idt)
+    x = ops.token_embed(ids.to(torch.int32), table)
+    got = ops.embed_rmsnorm(ids, table, w, 1e-5)
+    assert torch.equal(got[0], x) and got[0].shape == (rows, 1, N)
+    assert torch.equal(got[1], ops.rmsnorm(x, w, 1e-5)[0])
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
