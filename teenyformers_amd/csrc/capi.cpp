@@ -448,11 +448,17 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
     long total = (long)nmb * batch * (pack ? hkv : hq);
     if (total >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
     int tot = (int)total;
-    snprintf(name, sizeof name, "teeny_fa2_bwd_dq_bf16_d%d_%s%s%s", head_dim, cz,
-             pack ? "_g4" : "", gsfx);
+    // at most one workgroup a CU and a long walk: two wavefront groups share
+    // its keys (backward, 1 group against 2: B1 Hq8 Hkv2 S4096 D128 185 and
+    // 170 us, B1 Hq8 Hkv1 S3125 D128 140 and 131, B1 H16 S2048 D64 79 and 74,
+    // B1 Hq32 Hkv8 S1021 D64 53 and 51; shorter walks pay more for the second
+    // group's Q, dO and O rows: S1024 D128 equal, S300 D64 20.0 and 20.6)
+    const bool k2 = total <= device_cus() && n_ctx_k >= 15 * head_dim;
+    snprintf(name, sizeof name, "teeny_fa2_bwd_dq_bf16_d%d_%s%s%s%s", head_dim, cz,
+             pack ? "_g4" : "", k2 ? "_k2" : "", gsfx);
     void* a2[] = {&q,       &k,       &v,     &o,  &dout, &l,   &ld,  &dq,
                   &n_ctx_q, &n_ctx_k, &scale, &hq, &hkv,  &nmb, &tot};
-    rc = launch(name, dim3(tot), dim3(256), 0, stream, a2);
+    rc = launch(name, dim3(tot), dim3(k2 ? 512 : 256), 0, stream, a2);
     if (rc) return rc;
     // dK, dV: one workgroup per 128 keys of a (b, kv head) and share of the
     // group's q heads (a split needs the larger workspace; without it the

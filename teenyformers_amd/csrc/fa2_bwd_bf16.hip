@@ -154,8 +154,11 @@ __device__ __forceinline__ void fa2_bwd_dkdv(
   // the walk's (head, q-block) items it0 .. it0 + n_iter - 1: share hs of
   // hsplit (two groups: the whole walk)
   const int items = group * per_head;
-  const int it0 = NG == 1 ? (int)((long)items * hs / hsplit) : 0;
-  const int n_iter = NG == 1 ? (int)((long)items * (hs + 1) / hsplit) - it0 : items;
+  int it0 = 0, n_iter = items;
+  if (NG == 1 && hsplit > 1) {  // (the divisions cost a whole walk 0.5 us)
+    it0 = (int)((long)items * hs / hsplit);
+    n_iter = (int)((long)items * (hs + 1) / hsplit) - it0;
+  }
 
   // Q / dO tiles: chunk P = i*256 + tid of a tile holds tile chunk swz(P);
   // the swizzle repeats every 256 chunks.  Wave 0 also brings the rows'
@@ -481,8 +484,12 @@ struct __attribute__((aligned(16))) DqSmem {
 };
 
 // PACK: GQA groups of 4 packed as in the forward, one workgroup per (b, kv
-// head, 32 query rows), wavefront w on q head kv head * 4 + w
-template <int D, bool CAUSAL, typename GT, bool PACK = false>
+// head, 32 query rows), wavefront w on q head kv head * 4 + w.
+// KG = 2 (grids that leave a CU one workgroup of 4 wavefronts, one per SIMD,
+// whose walk over the keys is then a serial chain): two groups of 4 wavefronts
+// on the same rows, each on half of the key tiles in buffers of its own; group
+// 0 adds group 1's dQ (fp32, through LDS) to its own and stores it.
+template <int D, bool CAUSAL, typename GT, bool PACK = false, int KG = 1>
 __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ k,
                            const bf16* __restrict__ v, const bf16* __restrict__ o,
                            const bf16* __restrict__ dout, const float* __restrict__ lse,
@@ -494,14 +501,16 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
   constexpr int TILE = QBN * D * 2;    // bytes per tile
   constexpr int HALF = 32 * D * 2;     // bytes of 32 rows
   constexpr int TCH = QBN * CPR / 256; // 16-byte chunks per thread per tile
-  __shared__ DqSmem<D> sm;
+  __shared__ DqSmem<D> sms[KG];
 
   // fp32 gradients: dS also enters the dQ product as a second, low bf16 part
   // (dS = hi + lo), so its bf16 operand rounding drops from 2^-9 to 2^-17
   constexpr bool PRECISE = std::is_same<GT, float>::value;
-  const int tid = threadIdx.x;
-  // wave-uniform (an SGPR): every branch on it is a scalar branch
+  // within the group of 4 wavefronts
+  const int tid = KG == 1 ? threadIdx.x : threadIdx.x & 255;
+  // wave-uniform (SGPRs): every branch on them is a scalar branch
   const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
   const int l32 = lane & 31, g = lane >> 5;
 
   const int id = xcd_remap(blockIdx.x, total_blocks);
@@ -573,7 +582,7 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
       dlt = part;
     }
     const int nq_pad = (nq + BM - 1) / BM * BM;  // ld rows: whole blocks of BM
-    if (g == 0 && qrow < nq_pad) {
+    if ((KG == 1 || grp == 0) && g == 0 && qrow < nq_pad) {
       float* blk = ld + ((long)bhq * nq_pad + qrow) / BM * (2 * BM);
       blk[qrow % BM] = qok ? -lse[(long)bhq * nq + qrow] / scale : -INFINITY;
       blk[BM + qrow % BM] = -dlt;
@@ -583,19 +592,25 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
 
   int kend = nk;
   if (CAUSAL) kend = min(nk, blk_end);
-  const int n_iter = (kend + QBN - 1) / QBN;
-  // causal: the workgroup's tiles past this wavefront's last row are fully
-  // masked for it; it computes only the first n_live (wave-uniform)
-  const int n_live = CAUSAL ? min(n_iter, (wrow0 + 31) / QBN + 1) : n_iter;
+  const int n_all = (kend + QBN - 1) / QBN;
+  // the group's tiles: n_iter from tile0 (the second group may have one fewer
+  // than n_bar, the steps whose barriers both meet)
+  const int n_bar = (n_all + KG - 1) / KG, tile0 = grp * n_bar;
+  const int n_iter = KG == 1 ? n_all : min(n_bar, n_all - tile0);
+  // causal: the group's tiles past this wavefront's last row are fully masked
+  // for it; it computes only the first n_live (wave-uniform)
+  const int n_live =
+      KG == 1 ? (CAUSAL ? min(n_iter, (wrow0 + 31) / QBN + 1) : n_iter)
+              : (CAUSAL ? max(0, min(n_iter, (wrow0 + 31) / QBN + 1 - tile0)) : n_iter);
 
   // ---- K / V tiles: buffer_load ... lds, both SWZ_DUAL ----------------------
   const uint32_t src = swz<SWZ_DUAL, D>(wave * 64 + lane) * 16;
   const auto krsrc = make_rsrc(kb, nk * D * 2);
   const auto vrsrc = make_rsrc(vb, nk * D * 2);
   auto load_tile = [&](int it, int koff, int voff) {
-    const int kbase = it * QBN;
-    char* kdst = sm.k[0] + koff + wave * 64 * 16;
-    char* vdst = sm.v[0] + voff + wave * 64 * 16;
+    const int kbase = (KG == 1 ? it : tile0 + it) * QBN;
+    char* kdst = sms[KG == 1 ? 0 : grp].k[0] + koff + wave * 64 * 16;
+    char* vdst = sms[KG == 1 ? 0 : grp].v[0] + voff + wave * 64 * 16;
     const int sbase = kbase * D * 2;
     if (kbase + QBN <= nk) {
 #pragma unroll
@@ -744,7 +759,7 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
   // The first lagged product reads the K half "before" tile 0 with dS = 0:
   // zero it (buffer QKBUF-1, second half) so that 0 * K stays 0.
   for (int i = tid; i < HALF / 16; i += 256)
-    *reinterpret_cast<u32x4*>(sm.k[QKBUF - 1] + HALF + 16 * i) = u32x4{0, 0, 0, 0};
+    *reinterpret_cast<u32x4*>(sms[KG == 1 ? 0 : grp].k[QKBUF - 1] + HALF + 16 * i) = u32x4{0, 0, 0, 0};
   // tile 1 is requested with tile 0, before the first wait (its latency
   // overlaps tile 0's); the barrier alone, since __syncthreads would wait
   // for tile 1's loads too
@@ -766,12 +781,12 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
       f32x16 s, dp;
-      s_dp(sm.k[kb] + u * HALF, sm.v[vb] + u * HALF, s, dp);
+      s_dp(sms[KG == 1 ? 0 : grp].k[kb] + u * HALF, sms[KG == 1 ? 0 : grp].v[vb] + u * HALF, s, dp);
       if (u == 0 && it > 0 && it + 1 < n_iter)  // after the first products (as in the forward)
         load_tile(it + 1, ((kb + 1) % QKBUF) * TILE, ((vb + 1) % QVBUF) * TILE);
-      mask(it * QBN + 32 * u, s);
+      mask((KG == 1 ? it : tile0 + it) * QBN + 32 * u, s);
       // the pending dS^T is of the previous half: tile it-1's second half, then this tile's first
-      dq_and_ds(u == 0 ? sm.k[(kb + QKBUF - 1) % QKBUF] + HALF : sm.k[kb], s, dp);
+      dq_and_ds(u == 0 ? sms[KG == 1 ? 0 : grp].k[(kb + QKBUF - 1) % QKBUF] + HALF : sms[KG == 1 ? 0 : grp].k[kb], s, dp);
     }
     __builtin_amdgcn_s_waitcnt(0);  // this thread's loads of tile it+1 have landed
     __syncthreads();
@@ -794,15 +809,18 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
   if (it + 2 < n_live) tile_step(it + 2, I2{}, I0{});
   if (it + 3 < n_live) tile_step(it + 3, I0{}, I1{});
   if (it + 4 < n_live) tile_step(it + 4, I1{}, I0{});
-  if (n_iter > 0) {  // tile n_live-1's second half: its dS^T product is pending
-    const char* kl = sm.k[0] + ((n_live - 1) % QKBUF) * TILE + HALF;
+  if (KG == 2 || n_iter > 0) {
+    if (KG == 1 || n_live > 0) {  // tile n_live-1's second half: its dS^T product is pending
+      const char* kl = sms[KG == 1 ? 0 : grp].k[0] + ((n_live - 1) % QKBUF) * TILE + HALF;
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) dq_mfma(j, dq_read(kl, j));
+      for (int j = 0; j < NJ; ++j) dq_mfma(j, dq_read(kl, j));
+    }
     // a wavefront whose rows end before the workgroup's last tiles still
     // loads its share of them and meets the workgroup at each of their
     // barriers (tile t + 1 goes to K buffer (t + 1) % 3, V buffer (t + 1) % 2)
-    for (int t = n_live; t < n_iter; ++t) {
-      if (t + 1 < n_iter) load_tile(t + 1, ((t + 1) % QKBUF) * TILE, ((t + 1) % QVBUF) * TILE);
+    for (int t = n_live; t < (KG == 1 ? n_iter : n_bar); ++t) {
+      if ((KG == 1 || t > 0) && t + 1 < n_iter)
+        load_tile(t + 1, ((t + 1) % QKBUF) * TILE, ((t + 1) % QVBUF) * TILE);
       __builtin_amdgcn_s_waitcnt(0);
       __syncthreads();
     }
@@ -814,7 +832,28 @@ __device__ void fa2_bwd_dq(const bf16* __restrict__ q, const bf16* __restrict__ 
   __builtin_amdgcn_s_waitcnt(kVmWaitLgkm0<63>());
   barrier_only();
   (void)qok;
-  store_tile_rows<D, GT>(reinterpret_cast<char*>(&sm) + wave * (32 * D * (int)sizeof(GT)),
+  if constexpr (KG == 2) {
+    static_assert(sizeof(DqSmem<D>) >= 4 * 32 * D * 4, "group 1's dQ fits its buffers");
+    f32x4* part = reinterpret_cast<f32x4*>(&sms[1]) + wave * (DT * 4 * 64) + lane;
+    if (grp == 1)
+#pragma unroll
+      for (int t = 0; t < DT; ++t)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          part[(t * 4 + j) * 64] =
+              f32x4{acc[t][4 * j], acc[t][4 * j + 1], acc[t][4 * j + 2], acc[t][4 * j + 3]};
+    __syncthreads();
+    if (grp == 1) return;
+#pragma unroll
+    for (int t = 0; t < DT; ++t)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const f32x4 o = part[(t * 4 + j) * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][4 * j + e] += o[e];
+      }
+  }
+  store_tile_rows<D, GT>(reinterpret_cast<char*>(&sms) + wave * (32 * D * (int)sizeof(GT)),
                          dq + ((long)bhq * nq + wrow0) * D, nq - wrow0, [&](int t, int j) {
                            return f32x4{acc[t][4 * j] * scale, acc[t][4 * j + 1] * scale,
                                         acc[t][4 * j + 2] * scale, acc[t][4 * j + 3] * scale};
@@ -891,6 +930,27 @@ TEENY_FA2_BWD_DQ_G4_INST(64, bf16, )
 TEENY_FA2_BWD_DQ_G4_INST(128, bf16, )
 TEENY_FA2_BWD_DQ_G4_INST(64, float, _g32)
 TEENY_FA2_BWD_DQ_G4_INST(128, float, _g32)
+
+// dQ of small grids: two wavefront groups share a workgroup's keys (512
+// threads, one workgroup per CU)
+#define TEENY_FA2_BWD_DQ_K2_INST(D, CZ, CAUSAL, PACK, GT, SFX)                                   \
+  extern "C" __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))      \
+  void teeny_fa2_bwd_dq_bf16_d##D##_##CZ##_k2##SFX(                                             \
+      const bf16* q, const bf16* k, const bf16* v, const bf16* o, const bf16* dout,             \
+      const float* lse, float* ld, GT* dq, int nq, int nk, float scale, int hq, int hkv,        \
+      int nmb, int total) {                                                                     \
+    fa2_bwd_dq<D, CAUSAL, GT, PACK, 2>(q, k, v, o, dout, lse, ld, dq, nq, nk, scale, hq, hkv,  \
+                                       nmb, total);                                             \
+  }
+#define TEENY_FA2_BWD_DQ_K2(D)                              \
+  TEENY_FA2_BWD_DQ_K2_INST(D, c, true, false, bf16, )       \
+  TEENY_FA2_BWD_DQ_K2_INST(D, n, false, false, bf16, )      \
+  TEENY_FA2_BWD_DQ_K2_INST(D, c_g4, true, true, bf16, )     \
+  TEENY_FA2_BWD_DQ_K2_INST(D, c, true, false, float, _g32)  \
+  TEENY_FA2_BWD_DQ_K2_INST(D, n, false, false, float, _g32) \
+  TEENY_FA2_BWD_DQ_K2_INST(D, c_g4, true, true, float, _g32)
+TEENY_FA2_BWD_DQ_K2(64)
+TEENY_FA2_BWD_DQ_K2(128)
 
 extern "C" __global__ __launch_bounds__(256) void teeny_fa2_dkdv_merge_bf16(
     const float* part, bf16* dk, bf16* dv, long n, int hsplit, float scale) {

@@ -458,6 +458,31 @@ def test_fa2_bf16_bwd_shared_walk(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32)
         check_bf16(name, host(got), w)
 
 
+@pytest.mark.parametrize("grad_f32", [False, True])
+@pytest.mark.parametrize("B,Hq,Hkv,Sq,Sk,D,causal", [
+    (1, 2, 2, 1000, 1000, 64, True),   # blocks of 2 to 16 tiles of 64 keys
+    (1, 4, 1, 1025, 1025, 64, True),   # GQA groups of 4: blocks of one tile (none for group 1) to 17
+    (1, 1, 1, 33, 960, 64, False),     # 15 tiles, the shortest walk taken
+    (2, 2, 1, 1, 1023, 64, False),     # one row, a last tile of 63 keys
+    (1, 4, 1, 64, 1985, 128, True),    # one tile a block, keys past every row
+    (1, 1, 1, 1930, 1930, 128, True),
+    (1, 2, 2, 130, 1921, 128, False),  # 31 tiles, the last of one key
+])
+def test_fa2_bf16_bwd_dq_two_key_groups(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32):
+    """dQ whose keys two wavefront groups of a workgroup share (few rows, long
+    walks), against the oracle at the bf16 bar, twice with the same bits."""
+    q, k, v, do = inputs(67, B, Hq, Hkv, Sq, Sk, D, bf16=True)
+    scale = 1.0 / math.sqrt(D)
+    qd, kd, vd, dod = (dev(t, torch.bfloat16) for t in (q, k, v, do))
+    o, lse = ops.flash_attn2_fwd(qd, kd, vd, scale, causal)
+    a = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
+    b = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
+    assert all(torch.equal(x, y) for x, y in zip(a, b))
+    want = O.fa2_bwd(q, k, v, host(o), do, host(lse), scale, causal)
+    for name, got, w in zip(("dq", "dk", "dv"), a, want):
+        check_bf16(name, host(got), w)
+
+
 def _random_shapes(n, seed=2026):
     """Seeded random shapes off the tile grid: ragged lengths, Sq != Sk, GQA
     groups 1-8, both head dims."""
