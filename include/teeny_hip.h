@@ -98,6 +98,10 @@ int teeny_profile_kernel_names(char* buf, size_t buf_bytes);
  * neg_inf must be -INFINITY (the only value the reference passes,
  * flash_attn2.rs:478, :331).  softmax_scale: finite; > 0 for bf16 (the bf16
  * kernels fold the scale into the exponent after masking raw scores).
+ * A causally masked (query, key) pair has no influence.  fp32: whatever its
+ * rows hold.  bf16: it enters the products as 0 * V (0 * K, Q, dO in the
+ * backward), so those rows must be finite (rows at or past n_ctx are never
+ * read).
  * Backward dtype: TEENY_F32, TEENY_BF16 or TEENY_BF16 | TEENY_GRAD_F32.
  * ------------------------------------------------------------------------ */
 

@@ -183,6 +183,82 @@ def test_fa2_f32_edges(cuda, shape, causal, aligned):
         assert err <= F32_TOL * max(1.0, float(np.abs(want).max())), f"{name} {err}"
 
 
+@pytest.mark.parametrize("shape", [  # B, Hq, Hkv, Sq, Sk, D
+    (1, 1, 1, 40, 40, 64), (2, 4, 2, 100, 100, 128), (1, 2, 1, 70, 70, 32), (1, 2, 2, 37, 37, 16),
+    (1, 1, 1, 65, 65, 8),
+    (1, 2, 1, 50, 90, 64),     # keys past every query row
+    (1, 8, 1, 200, 70, 64),    # the dK/dV walk shared out over workgroups
+])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_fa2_f32_causal_masked_rows_are_inert(cuda, shape, bad):
+    """A causally masked (query, key) pair has no influence, whatever its rows
+    hold: with K and V not finite from key n on, query rows before n keep the
+    O, LSE and dQ of finite K and V; with Q, dO and LSE not finite before
+    query n, keys from n on keep their dK and dV.  n falls inside the 32-row
+    tiles, at their edges and at the 16-row wavefronts'."""
+    B, Hq, Hkv, Sq, Sk, D = shape
+    q, k, v, do = inputs(40, *shape, bf16=False)
+    scale = 1.0 / math.sqrt(D)
+    oe, le = O.fa2_fwd(q, k, v, scale, True)
+    want = O.fa2_bwd(q, k, v, oe, do, le, scale, True)
+
+    def same(name, n, got, exact):
+        got = host(got)
+        assert np.isfinite(got).all(), f"{name} n={n}"
+        bar = F32_TOL * max(1.0, float(np.abs(exact).max()))
+        assert np.abs(got - exact).max() <= bar, f"{name} n={n}"
+
+    put = lambda t: dev(t, torch.float32)  # noqa: E731
+    qd, kd, vd, dod, od, lsed = (put(t) for t in (q, k, v, do, oe, le))
+    for n in (1, 7, 16, 31, 32, 33, min(Sq, Sk) - 1, min(Sq, Sk)):
+        kb, vb = kd.clone(), vd.clone()
+        kb[:, :, n:] = vb[:, :, n:] = bad
+        o, lse = ops.flash_attn2_fwd(qd, kb, vb, scale, True)
+        dq, _, _ = ops.flash_attn2_bwd(qd, kb, vb, od, lsed, dod, scale, True)
+        same("o", n, o[:, :, :n], oe[:, :, :n])
+        same("lse", n, lse.view(B, Hq, Sq)[:, :, :n], le.reshape(B, Hq, Sq)[:, :, :n])
+        same("dq", n, dq[:, :, :n], want[0][:, :, :n])
+        qb, dob, lb = qd.clone(), dod.clone(), lsed.clone()
+        qb[:, :, :n] = dob[:, :, :n] = bad
+        lb.view(B, Hq, Sq)[:, :, :n] = bad
+        _, dk, dv = ops.flash_attn2_bwd(qb, kd, vd, od, lb, dob, scale, True)
+        if n < Sk:
+            same("dk", n, dk[:, :, n:], want[1][:, :, n:])
+            same("dv", n, dv[:, :, n:], want[2][:, :, n:])
+
+
+@pytest.mark.parametrize("causal", [True, False])
+@pytest.mark.parametrize("D", [32, 64, 128])
+def test_fa2_f32_visible_infinities(cuda, causal, D):
+    """One infinite V element reaches its own column of the rows that see it
+    and nothing else, in a tile on the diagonal as elsewhere; a key whose
+    score is -inf for every query (an infinite K element against queries of
+    one sign) has dK = dV = 0, also where the last query tile is ragged."""
+    B, H, S, r, d = 1, 2, 77, 41, 5
+    q, k, v, do = inputs(44, B, H, H, S, S, D, bf16=False)
+    scale = 1.0 / math.sqrt(D)
+    oe, le = O.fa2_fwd(q, k, v, scale, causal)
+    vb = v.copy()
+    vb[:, :, r, d] = np.inf
+    o, lse = ops.flash_attn2_fwd(*(dev(t, torch.float32) for t in (q, k, vb)), scale, causal)
+    o = host(o)
+    sees = np.arange(S) >= (r if causal else 0)
+    assert np.isposinf(o[:, :, sees, d]).all()
+    o[:, :, sees, d] = oe[:, :, sees, d]
+    assert np.abs(o - oe).max() <= F32_TOL
+    assert np.abs(host(lse).reshape(le.shape) - le).max() <= F32_TOL
+    q[..., 0] = np.abs(q[..., 0]) + 0.125
+    kb = k.copy()
+    kb[:, :, r, 0] = -np.inf
+    keep = np.arange(S) != r
+    qd, kd, vd, dod = (dev(t, torch.float32) for t in (q, kb, v, do))
+    o, lse = ops.flash_attn2_fwd(qd, kd, vd, scale, causal)
+    assert torch.isfinite(o).all() and torch.isfinite(lse).all()
+    _, dk, dv = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal)
+    assert not dk[:, :, r].any() and not dv[:, :, r].any()
+    assert torch.isfinite(dk[:, :, keep]).all() and torch.isfinite(dv[:, :, keep]).all()
+
+
 # ---------------------------------------------------------------------------
 # bf16 MFMA path
 # ---------------------------------------------------------------------------
