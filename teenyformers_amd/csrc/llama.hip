@@ -346,7 +346,8 @@ __device__ __forceinline__ void decode_f32(const float* __restrict__ q,
   zero_acc<D>(acc);
   float m = -INFINITY, l = 0.0f;
   for (int t0 = k0; t0 < k1; t0 += 32) {
-    // rows at or past k1 re-read row k1 - 1; their P is zero
+    // rows at or past k1 re-read row k1 - 1; their P is zero, and so is their V
+    // below (0 * an infinite V of that row is NaN)
     f32x4 kf[2][NC];
     float vf[8][NH][VW];
 #pragma unroll
@@ -400,6 +401,15 @@ __device__ __forceinline__ void decode_f32(const float* __restrict__ q,
     for (int h = 0; h < NH; ++h)
 #pragma unroll
       for (int e = 0; e < VW; ++e) acc[h][e] *= alpha;
+    if (t0 + 32 > k1) {
+#pragma unroll
+      for (int x = 0; x < 8; ++x)
+        if (t0 + 16 * (x >> 2) + 4 * g + (x & 3) >= k1)
+#pragma unroll
+          for (int h = 0; h < NH; ++h)
+#pragma unroll
+            for (int e = 0; e < VW; ++e) vf[x][h][e] = 0.0f;
+    }
 #pragma unroll
     for (int x = 0; x < 8; ++x)
 #pragma unroll

@@ -293,6 +293,21 @@ def test_decode_attention_f32_edges(cuda, B, Hq, Hkv, D, n_keys, L):
     assert (o.double() - want).abs().max().item() <= 1e-5
 
 
+@pytest.mark.parametrize("D,n_keys", [(64, 1), (64, 45), (128, 97), (32, 63), (8, 33)])
+def test_decode_attention_f32_last_key_infinite(cuda, D, n_keys):
+    """An infinite V element of the last key, which lies inside a 32-key tile,
+    gives its column infinity and leaves the others as they are."""
+    g = torch.Generator(device="cuda").manual_seed(n_keys)
+    q = torch.randn(2, 4, D, generator=g, device="cuda")
+    k, v = (torch.randn(2, 2, n_keys + 3, D, generator=g, device="cuda") for _ in range(2))
+    want = ops.decode_attention(q, k, v, n_keys)
+    v[:, :, n_keys - 1, 3] = float("inf")
+    got = ops.decode_attention(q, k, v, n_keys)
+    assert torch.isposinf(got[..., 3]).all()
+    keep = torch.arange(D, device="cuda") != 3
+    assert torch.equal(got[..., keep], want[..., keep])
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,L", [
     (4, 32, 8, 128, 640),   # the Llama-3-8B decode shape
     (3, 8, 1, 64, 300),     # 8 q heads on one kv head, cache off the 32-key tile
