@@ -378,7 +378,7 @@ __device__ __forceinline__ void decode_f32(const float* __restrict__ q,
       for (int e = 0; e < 4; ++e)
 #pragma unroll
         for (int u = 0; u < 2; ++u) s[u] = mfma4(kf[u][c][e], qf[c][e], s[u]);
-    float mx = -INFINITY;
+    float mx = -INFINITY, m_old = m;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
@@ -386,15 +386,15 @@ __device__ __forceinline__ void decode_f32(const float* __restrict__ q,
         s[u][r] = t0 + 16 * u + 4 * g + r < k1 ? s[u][r] * scale : -INFINITY;
         mx = fmaxf(mx, s[u][r]);
       }
-    const float m_new = fmaxf(m, max_g(mx));  // the tile has a key below k1
-    const float alpha = expf(m - m_new);
-    m = m_new;
+    m = fmaxf(m, max_g(mx));
+    const float ref = m == -INFINITY ? 0.0f : m;  // every score so far -inf: P = 0
+    const float alpha = expf(m_old - ref);
     l *= alpha;
 #pragma unroll
     for (int u = 0; u < 2; ++u)
 #pragma unroll
       for (int r = 0; r < 4; ++r) {
-        s[u][r] = expf(s[u][r] - m_new);
+        s[u][r] = expf(s[u][r] - ref);
         l += s[u][r];
       }
 #pragma unroll

@@ -308,6 +308,24 @@ def test_decode_attention_f32_last_key_infinite(cuda, D, n_keys):
     assert torch.equal(got[..., keep], want[..., keep])
 
 
+@pytest.mark.parametrize("lo,hi", [(0, 32), (0, 64), (32, 64), (64, 128), (0, 129)])
+def test_decode_attention_f32_masked_tiles(cuda, lo, hi):
+    """Keys lo .. hi - 1 with a score of -inf (an infinite K element against
+    queries of one sign), whole 32-key tiles and key splits of them: the
+    result is that of the other keys."""
+    D, n_keys = 64, 130
+    g = torch.Generator(device="cuda").manual_seed(lo + hi)
+    q = torch.randn(2, 4, D, generator=g, device="cuda")
+    q[..., 0] = q[..., 0].abs() + 0.125
+    k, v = (torch.randn(2, 2, n_keys, D, generator=g, device="cuda") for _ in range(2))
+    k[:, :, lo:hi, 0] = -float("inf")
+    got = ops.decode_attention(q, k, v, n_keys)
+    keep = [i for i in range(n_keys) if not lo <= i < hi]
+    kk, vv = (t[:, :, keep].double().repeat_interleave(2, 1) for t in (k, v))
+    p = ((kk * q.double()[:, :, None]).sum(-1) / D ** 0.5).softmax(-1)
+    assert (got.double() - (p[..., None] * vv).sum(2)).abs().max().item() <= 1e-5
+
+
 @pytest.mark.parametrize("B,Hq,Hkv,D,L", [
     (4, 32, 8, 128, 640),   # the Llama-3-8B decode shape
     (3, 8, 1, 64, 300),     # 8 q heads on one kv head, cache off the 32-key tile
