@@ -286,10 +286,12 @@ class Llama:
         """Whether a one-token step runs teeny_decode_qkv_attention_dev: bf16
         K-split QKV slabs, D 64 or 128, up to 32 q heads per kv head, and a
         cache short enough for one workgroup per (b, kv head), or few enough
-        of them that several share its keys."""
+        of them that several share its keys (a head's slab below 2 GiB: the
+        kernel's byte offsets are 32-bit)."""
         cfg = self.cfg
         return (isinstance(qkv, ops.Partials) and qkv.dtype == torch.bfloat16
                 and cfg.head_dim() in (64, 128) and cfg.n_heads // cfg.n_kv_heads() <= 32
+                and cache.capacity * cfg.head_dim() * 2 < 2 ** 31
                 and (cache.capacity <= 4096
                      or ops.decode_qkv_splits(qkv.shape[0], cfg.n_kv_heads(), cache.capacity) > 1))
 

@@ -358,3 +358,20 @@ def test_rope_base_tensor_by_value():
     first = ops._ln(base)
     base.fill_(5e5)
     assert first == ops._ln(1e4) and ops._ln(base) == ops._ln(5e5) != first
+
+
+def test_fused_decode_cache_limit(monkeypatch):
+    """A one-token step over a cache slab that the fused decode attention does
+    not address (2 GiB of one kv head) takes the unfused path, however many
+    workgroups would share its keys."""
+    from types import SimpleNamespace
+
+    import torch
+
+    from teenyformers_amd import llama, ops
+    cfg = llama.LlamaConfig(d_model=512, n_heads=4, n_kv_heads_=1)
+    model = llama.Llama(cfg, {})
+    qkv = ops.Partials(torch.empty(1, 1, 768), (1, 1, 768), torch.bfloat16)
+    monkeypatch.setattr(ops, "decode_qkv_splits", lambda *a: 16)
+    assert model._fused_decode(qkv, SimpleNamespace(capacity=8_388_607))
+    assert not model._fused_decode(qkv, SimpleNamespace(capacity=8_388_608))
