@@ -1319,10 +1319,11 @@ int teeny_gemm_bf16(const void* x, const void* w, void* y, int M, int N, int K,
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
   if (M <= 0 || N <= 0 || K <= 0 || (long)N * K >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
   if (N % 64 != 0 || K % 64 != 0) return TEENY_ERR_UNSUPPORTED;
+  // a workgroup addresses its 256 rows of x and of w with 32-bit byte offsets
+  // (the K that the entry point takes, at any M)
+  if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   if (M <= 64 && N % 128 == 0 && K % 128 == 0)
     return launch_linear_rows(x, w, y, M, N, K, TEENY_LINEAR_PLAIN, K, 0, stream);
-  // a workgroup addresses its 256 rows of x and of w with 32-bit byte offsets
-  if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   int tiles_m = (M + 255) / 256, tiles_n = (N + 255) / 256;
   if ((long)tiles_m * tiles_n >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   void* args[] = {&x, &w, &y, &M, &N, &K, &tiles_m, &tiles_n};
@@ -1403,10 +1404,11 @@ int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F
                              hipStream_t stream) {
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
   if (M <= 0 || F <= 0 || K <= 0 || 2L * F * K >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
-  if (M <= 64 && F % 64 == 0 && K % 128 == 0)
-    return launch_linear_rows(x, w, y, M, F, K, TEENY_LINEAR_SWIGLU, K, 0, stream);
+  const bool rows = F % 64 == 0 && K % 128 == 0;
+  if (M <= 16 && rows) return launch_linear_rows(x, w, y, M, F, K, TEENY_LINEAR_SWIGLU, K, 0, stream);
   if (F % 32 != 0 || K % 64 != 0) return TEENY_ERR_UNSUPPORTED;
   if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
+  if (M <= 64 && rows) return launch_linear_rows(x, w, y, M, F, K, TEENY_LINEAR_SWIGLU, K, 0, stream);
   int tiles_m = (M + 255) / 256, tiles_n = (F + 127) / 128;
   if ((long)tiles_m * tiles_n >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   void* args[] = {&x, &w, &y, &M, &F, &K, &tiles_m, &tiles_n};

@@ -208,6 +208,10 @@ def test_decode_ops_validation(L):
     assert L.teeny_linear_swiglu_bf16(P, P, P, 17, 48, 128, None) == UNSUP
     assert L.teeny_linear_swiglu_bf16(P, P, P, 300, 64, 96, None) == UNSUP
     assert L.teeny_linear_swiglu_bf16(P, P, P, 300, 64, 1 << 22, None) == SHAPE
+    # the same K limit where 17 to 64 rows stream the weight
+    assert L.teeny_linear_swiglu_bf16(P, P, P, 64, 64, 1 << 22, None) == SHAPE
+    for m in (4, 64, 300):
+        assert L.teeny_gemm_bf16(P, P, P, m, 128, 1 << 22, None) == SHAPE
     assert L.teeny_linear_swiglu_bf16(P, None, P, 300, 64, 128, None) == NULLP
     assert L.teeny_linear_bf16(None, P, P, 16, 128, 128, None) == NULLP
     assert L.teeny_linear_bf16(P, P, P, 0, 128, 128, None) == SHAPE
