@@ -1266,6 +1266,7 @@ int teeny_argmax_rows_advance(const void* x, int64_t* out, int rows, int cols, i
 
 // Decode-step linear layers (linear_bf16.hip): 512 threads, 128 W rows per
 // workgroup (64 gate + 64 up rows for SwiGLU), x staged in 512-wide K chunks.
+// The shapes of the entry points for up to 16 rows:
 static int linear_sk_check(const void* x, const void* w, const void* y, int M, int N, int K,
                            long w_rows, int row_tile) {
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
@@ -1274,7 +1275,8 @@ static int linear_sk_check(const void* x, const void* w, const void* y, int M, i
   return TEENY_OK;
 }
 
-// The same kernels for up to 64 rows: tiles of 16 x rows, 1, 2 or 4 of them.
+// The one launch of them all, up to 64 rows: tiles of 16 x rows, 1, 2 or 4 of
+// them.
 static int launch_linear_rows(const void* x, const void* w, void* y, int M, int N, int K, int op,
                               int k_split, int layout, hipStream_t stream) {
   const char* mt = M <= 16 ? "" : M <= 32 ? "_m2" : "_m4";
@@ -1338,10 +1340,8 @@ int teeny_linear_bf16(const void* x, const void* w, void* y, int M, int N, int K
                       hipStream_t stream) {
   if (!x || !w || !y) return TEENY_ERR_NULL_POINTER;
   if (M <= 0 || N <= 0 || K <= 0 || (long)N * K >= kMaxElems * 2) return TEENY_ERR_INVALID_SHAPE;
-  if (M <= 16 && N % 128 == 0 && K % 128 == 0) {
-    void* args[] = {&x, &w, &y, &M, &N, &K};
-    return launch("teeny_linear_sk_bf16", dim3(N / 128), dim3(512), 0, stream, args);
-  }
+  if (M <= 16 && N % 128 == 0 && K % 128 == 0)
+    return launch_linear_rows(x, w, y, M, N, K, TEENY_LINEAR_PLAIN, K, 0, stream);
   if (N % 64 != 0 || K % 64 != 0) return TEENY_ERR_UNSUPPORTED;
   if ((long)K * 2 * 256 >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
   if (M > 16 && teeny_lt_gemm_bf16(x, w, y, M, N, K, stream) == 0) return TEENY_OK;
@@ -1424,14 +1424,8 @@ int teeny_linear_partials_count(int K, int k_split) {
 int teeny_linear_partials_bf16(const void* x, const void* w, float* parts, int M, int N, int K,
                                int k_split, hipStream_t stream) {
   int rc = linear_sk_check(x, w, parts, M, N, K, N, 128);
-  if (rc) return rc;
-  if (k_split <= 0) return TEENY_ERR_INVALID_VALUE;
-  if (k_split >= K) k_split = K;
-  else if (k_split % 128 != 0) return TEENY_ERR_INVALID_VALUE;  // whole 128-wide K steps
-  const int n = teeny_linear_partials_count(K, k_split);
-  if (n > 65535) return TEENY_ERR_INVALID_SHAPE;
-  void* args[] = {&x, &w, &parts, &M, &N, &K, &k_split};
-  return launch("teeny_linear_sk_part_bf16", dim3(N / 128, n), dim3(512), 0, stream, args);
+  return rc ? rc : teeny_linear_rows_bf16(x, w, parts, M, N, K, TEENY_LINEAR_PARTIALS, k_split, 0,
+                                          stream);
 }
 
 // The streaming layout of a decode weight (linear_bf16.hip): a copy of W in
@@ -1456,30 +1450,20 @@ int teeny_linear_stream_layout_bf16(const void* w, void* w_s, int N, int K, hipS
 int teeny_linear_sl_bf16(const void* x, const void* w_s, void* y, int M, int N, int K,
                          hipStream_t stream) {
   int rc = linear_sk_check(x, w_s, y, M, N, K, N, 128);
-  if (rc) return rc;
-  void* args[] = {&x, &w_s, &y, &M, &N, &K};
-  return launch("teeny_linear_sl_bf16", dim3(N / 128), dim3(512), 0, stream, args);
+  return rc ? rc : teeny_linear_rows_bf16(x, w_s, y, M, N, K, TEENY_LINEAR_PLAIN, K, 1, stream);
 }
 
 int teeny_linear_swiglu_sl_bf16(const void* x, const void* w_s, void* y, int M, int F, int K,
                                 hipStream_t stream) {
   int rc = linear_sk_check(x, w_s, y, M, F, K, 2L * F, 64);
-  if (rc) return rc;
-  void* args[] = {&x, &w_s, &y, &M, &F, &K};
-  return launch("teeny_linear_sl_swiglu_bf16", dim3(F / 64), dim3(512), 0, stream, args);
+  return rc ? rc : teeny_linear_rows_bf16(x, w_s, y, M, F, K, TEENY_LINEAR_SWIGLU, K, 1, stream);
 }
 
 int teeny_linear_partials_sl_bf16(const void* x, const void* w_s, float* parts, int M, int N,
                                   int K, int k_split, hipStream_t stream) {
   int rc = linear_sk_check(x, w_s, parts, M, N, K, N, 128);
-  if (rc) return rc;
-  if (k_split <= 0) return TEENY_ERR_INVALID_VALUE;
-  if (k_split >= K) k_split = K;
-  else if (k_split % 128 != 0) return TEENY_ERR_INVALID_VALUE;  // whole 128-wide K steps
-  const int n = teeny_linear_partials_count(K, k_split);
-  if (n > 65535) return TEENY_ERR_INVALID_SHAPE;
-  void* args[] = {&x, &w_s, &parts, &M, &N, &K, &k_split};
-  return launch("teeny_linear_sl_part_bf16", dim3(N / 128, n), dim3(512), 0, stream, args);
+  return rc ? rc : teeny_linear_rows_bf16(x, w_s, parts, M, N, K, TEENY_LINEAR_PARTIALS, k_split, 1,
+                                          stream);
 }
 
 int teeny_token_embed_fwd(const void* ids, const void* weight, void* out, int seq_len,

@@ -443,6 +443,33 @@ def test_linear_stream_layout_bit_exact(cuda, M, N, K, k_split):
     assert p_sl.n == p_rm.n and torch.equal(p_sl.slabs, p_rm.slabs)
     if N % 128 == 0:  # F = N / 2, a multiple of 64
         assert torch.equal(ops.linear_swiglu(x, sw), ops.linear_swiglu(x, w))
+    # the entry points for up to 16 rows, and the one for up to 64
+    call, stream = ops._lib.call, torch.cuda.current_stream().cuda_stream
+    p = lambda t: t.data_ptr()  # noqa: E731
+    plain, swiglu, parts = (ops._lib.TEENY_LINEAR_PLAIN, ops._lib.TEENY_LINEAR_SWIGLU,
+                            ops._lib.TEENY_LINEAR_PARTIALS)
+    ks = K if k_split is None else k_split
+    n = ops._lib.lib().teeny_linear_partials_count(K, ks)
+    for layout, src in ((0, w), (1, sw.s)):
+        y, yr = (torch.empty(M, N, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+        s, sr = (torch.empty(n, M, N, device="cuda") for _ in range(2))
+        call("teeny_linear_rows_bf16", p(x), p(src), p(yr), M, N, K, plain, K, layout, stream)
+        call("teeny_linear_sl_bf16" if layout else "teeny_linear_bf16", p(x), p(src), p(y), M, N, K,
+             stream)
+        call("teeny_linear_rows_bf16", p(x), p(src), p(sr), M, N, K, parts, ks, layout, stream)
+        call("teeny_linear_partials_sl_bf16" if layout else "teeny_linear_partials_bf16", p(x),
+             p(src), p(s), M, N, K, ks, stream)
+        assert torch.equal(y, yr) and torch.equal(s, sr)
+        assert torch.equal(y, ops.linear(x, w))
+        if k_split is not None:
+            assert torch.equal(s, p_rm.slabs)
+        if N % 128 == 0:
+            f, fr = (torch.empty(M, N // 2, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+            call("teeny_linear_rows_bf16", p(x), p(src), p(fr), M, N // 2, K, swiglu, K, layout,
+                 stream)
+            call("teeny_linear_swiglu_sl_bf16" if layout else "teeny_linear_swiglu_bf16", p(x),
+                 p(src), p(f), M, N // 2, K, stream)
+            assert torch.equal(f, fr) and torch.equal(f, ops.linear_swiglu(x, w))
     # more than 16 rows: the row-major weight (the GEMM), same as without it
     x20 = torch.randn(20, K, device="cuda", generator=g).to(torch.bfloat16)
     assert torch.equal(ops.linear(x20, sw), ops.linear(x20, w))
