@@ -607,7 +607,8 @@ def _no_grad(x2: torch.Tensor, w: torch.Tensor) -> bool:
 def _skinny(x2: torch.Tensor, w: torch.Tensor, n_out: int, row_tile: int = 128,
             rows: int | None = None) -> bool:
     """Shapes the decode-step linear kernels take: up to 16 rows, and up to 64
-    within own_gemm() (other products of 17 rows or more go to hipBLASLt)."""
+    within own_gemm() or under capture (other products of 17 rows or more go
+    to hipBLASLt)."""
     M, K = x2.shape
     if rows is None:
         rows = split_rows()
@@ -636,8 +637,9 @@ _own_gemm = threading.local()
 def own_gemm():
     """Within this block, products run this library's GEMMs instead of
     hipBLASLt: bf16 products of 17 to 64 rows the weight-streaming decode
-    kernels, of more rows teeny_gemm_bf16, fp32 products teeny_gemm_f32.  That is the rule a captured graph follows by
-    itself (the linear entry points never run hipBLASLt under capture),
+    kernels, of more rows teeny_gemm_bf16, fp32 products teeny_gemm_f32.
+    That is the rule a captured graph follows by itself (the linear entry
+    points never run hipBLASLt under capture, and split_rows() is the same),
     applied to eager calls so that an eager step and its graph replay run
     the same kernels."""
     prev = getattr(_own_gemm, "on", False)
@@ -650,8 +652,11 @@ def own_gemm():
 
 def split_rows() -> int:
     """The row count up to which a model's products are taken as linear_split's
-    Partials: 64 within own_gemm() (decode steps), 16 otherwise (short prompts)."""
-    return 64 if getattr(_own_gemm, "on", False) else 16
+    Partials: 64 within own_gemm() (decode steps) and under graph capture, 16
+    otherwise (short prompts)."""
+    own = getattr(_own_gemm, "on", False) or (
+        torch.cuda.is_initialized() and torch.cuda.is_current_stream_capturing())
+    return 64 if own else 16
 
 
 class StreamWeight:

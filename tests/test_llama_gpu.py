@@ -394,6 +394,35 @@ def test_generate_graph_equals_eager(cuda, dtype, batch):
     assert torch.equal(eager, graph), (eager, graph)
 
 
+@pytest.mark.parametrize("batch", [3, 17, 64])
+def test_captured_hidden_equals_decode_step(cuda, batch):
+    """A one-token step that the caller captures by itself (no own_gemm()) has
+    the bits of decode_step: under capture the products follow the same rule."""
+    cfg = llama.LlamaConfig(d_model=512, n_heads=8, n_layers=2, vocab_size=512, eps=1e-5,
+                            rope_base=1e4, intermediate_size=1024, n_kv_heads_=2)
+    model = llama.Llama(cfg, llama.init_weights(cfg, dtype=torch.bfloat16, std=0.2, seed=31))
+    g = torch.Generator(device="cuda").manual_seed(32)
+    ids = torch.randint(0, 512, (batch, 9), generator=g, device="cuda")
+    cache, _ = model.prefill(ids, 16)
+    step = ids[:, -1:].contiguous()
+    want = model.decode_step(cache, step)  # writes row 9; the captured step writes it again
+    pos = torch.full((1,), 9, dtype=torch.int32, device="cuda")
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side), ops.own_gemm():
+        model.logits(model.hidden(step, cache, pos)[:, -1])
+    torch.cuda.current_stream().wait_stream(side)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = model.logits(model.hidden(step, cache, pos)[:, -1])
+    for _ in range(3):
+        got.fill_(float("nan"))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(got, want)
+
+
 def test_generate_stream_layout_equals_row_major(cuda):
     """Greedy ids of the graph-replayed decode with the weights in the
     streaming layout (ops.StreamWeight) == the eager decode from the
