@@ -1144,10 +1144,11 @@ int teeny_decode_qkv_attention_split_dev(const float* parts, int n_parts, void* 
     po = (float*)((char*)workspace + 2 * align256(rows * sizeof(float)));
   }
   char name[48];
-  snprintf(name, sizeof name, "teeny_decode_qkv_attn_bf16_d%d", head_dim);
+  snprintf(name, sizeof name, "teeny_decode_qkv_attn_%sbf16_d%d", n_split > 1 ? "split_" : "",
+           head_dim);
   void* args[] = {&parts,      &n_parts,   &part_stride, &k_cache,      &v_cache,
                   &o,          &n_heads_q, &n_heads_kv,  &n_past,       &cache_len,
-                  &ln_rope_base, &softmax_scale, &pm,    &pl,           &po};
+                  &ln_rope_base, &softmax_scale, &pm,    &pl,           &po};  // the last: split
   rc = launch(name, dim3((unsigned)(batch * n_heads_kv), (unsigned)n_split), dim3(512), 0, stream,
               args);
   if (rc || n_split == 1) return rc;

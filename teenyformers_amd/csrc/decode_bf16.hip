@@ -197,10 +197,13 @@ __device__ void decode_mfma(const bf16* __restrict__ q, const bf16* __restrict__
 //   3. the 8 partials (max, sum, unnormalised O) are merged in LDS and
 //      o [B, Hq, D] is stored, and the new k, v row is written to the cache
 //      (row n_past, when it is below cache_len) for the next steps.
-// gridDim.y > 1 (long caches, few sequences: B * Hkv workgroups would leave
-// most CUs idle): the keys are shared by that many such workgroups of a
-// (b, kv head), each repeating step 1, and the partials go to pm, pl, po for
-// teeny_decode_attn_combine (the host's rule and its figures: capi.cpp).
+// SPLIT (long caches, few sequences: B * Hkv workgroups would leave most CUs
+// idle): the keys are shared by gridDim.y such workgroups of a (b, kv head),
+// each repeating step 1, and the partials go to pm, pl, po for
+// teeny_decode_attn_combine (the host's rule and its figures: capi.cpp).  An
+// instance of its own: a share count read by the kernel took the unsplit step
+// from 4.7 to 5.0 us (2 sequences, 4 kv heads of 64, 21 keys), and 10.4 to 10.6
+// (16 sequences, 8 of 128, 521 keys).
 // It replaces the QKV split, the split-K decode kernel and the combine
 // kernel of the unfused path with one launch and no partials in HBM.
 constexpr int kDqWaves = 8;
@@ -223,7 +226,7 @@ struct __attribute__((aligned(16))) DecQkvSmem {
   float cs[D / 2][2];  // (cos, sin) of the pair angles at the new position
 };
 
-template <int D>
+template <int D, bool SPLIT>
 __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, long part_stride,
                                 bf16* __restrict__ kc, bf16* __restrict__ vc,
                                 bf16* __restrict__ o, int hq, int hkv,
@@ -245,7 +248,7 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
   const int n_keys = __builtin_amdgcn_readfirstlane(min(pos + 1, cache_len));
 
   // this wavefront's keys k0 .. k1 - 1, in 32-key tiles through its LDS buffer
-  const int n_split = gridDim.y, split = blockIdx.y;
+  const int n_split = SPLIT ? gridDim.y : 1, split = SPLIT ? blockIdx.y : 0;
   const int waves = kDqWaves * n_split;  // that share the keys
   const int kpw = ((n_keys + waves - 1) / waves + TK - 1) / TK * TK;
   const int k0 = (split * kDqWaves + wave) * kpw;
@@ -457,7 +460,7 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
     float mm = -INFINITY;
 #pragma unroll
     for (int w = 0; w < kDqWaves; ++w) mm = fmaxf(mm, sm.u.c.m[w][hh]);
-    const float ref = mm == -INFINITY ? 0.0f : mm;  // a split may have no keys
+    const float ref = SPLIT && mm == -INFINITY ? 0.0f : mm;  // a split may have no keys
     float num = 0.0f, den = 0.0f;
 #pragma unroll
     for (int w = 0; w < kDqWaves; ++w) {
@@ -466,7 +469,7 @@ __device__ void decode_qkv_attn(const float* __restrict__ parts, int n_parts, lo
       den += e * sm.u.c.l[w][hh];
     }
     const long row = (long)b * hq + hk * group + hh;
-    if (n_split == 1) {
+    if (!SPLIT) {
       o[row * D + d] = (bf16)(num / den);
     } else {
       const long r = row * n_split + split;
@@ -503,10 +506,16 @@ TEENY_DECODE_BF16_INST(128)
 #define TEENY_DECODE_QKV_INST(D)                                                                 \
   extern "C" __global__ __launch_bounds__(512) void teeny_decode_qkv_attn_bf16_d##D(            \
       const float* parts, int n_parts, long part_stride, bf16* kc, bf16* vc, bf16* o, int hq,    \
+      int hkv, const int* n_past, int cache_len, float ln_base, float scale) {                   \
+    decode_qkv_attn<D, false>(parts, n_parts, part_stride, kc, vc, o, hq, hkv, n_past,           \
+                              cache_len, ln_base, scale, nullptr, nullptr, nullptr);             \
+  }                                                                                              \
+  extern "C" __global__ __launch_bounds__(512) void teeny_decode_qkv_attn_split_bf16_d##D(      \
+      const float* parts, int n_parts, long part_stride, bf16* kc, bf16* vc, bf16* o, int hq,    \
       int hkv, const int* n_past, int cache_len, float ln_base, float scale, float* pm,          \
       float* pl, float* po) {                                                                    \
-    decode_qkv_attn<D>(parts, n_parts, part_stride, kc, vc, o, hq, hkv, n_past, cache_len,      \
-                       ln_base, scale, pm, pl, po);                                              \
+    decode_qkv_attn<D, true>(parts, n_parts, part_stride, kc, vc, o, hq, hkv, n_past, cache_len, \
+                             ln_base, scale, pm, pl, po);                                        \
   }
 
 TEENY_DECODE_QKV_INST(64)
