@@ -903,9 +903,14 @@ static int norm_bwd_impl(bool ref_formula, const void* dy, const void* h, void* 
   if (!workspace || workspace_bytes < teeny_fused_add_rmsnorm_bwd_workspace_bytes(M, N))
     return TEENY_ERR_WORKSPACE;
   // workgroups of 16, 8 or 4 wavefronts (bwd_waves in norm.hip), a row each
-  // at a time; one dweight partial per workgroup
+  // at a time; one dweight partial per workgroup.  Up to 64 rows 4 wavefronts,
+  // which spreads them over CUs, and at most 16 partials (bf16 with dweight
+  // given, full workgroups and the large reduction against this: 1 x 1000 6.5
+  // and 5.6 us, 16 x 2048 10.3 and 7.2, 64 x 4096 12.5 and 10.3)
   const int b = ch * vec * (int)dtype_size(dtype);
-  const int waves = b > 128 ? 4 : b > 64 || (vec == 1 && ch == 16) ? 8 : 16;
+  const int full = b > 128 ? 4 : b > 64 || (vec == 1 && ch == 16) ? 8 : 16;
+  const bool few = M <= 64;
+  const int waves = few ? 4 : full;
   int parts = (M + waves - 1) / waves;
   if (parts > kNormBwdMaxParts) parts = kNormBwdMaxParts;
   float* part = (float*)workspace;
@@ -916,9 +921,10 @@ static int norm_bwd_impl(bool ref_formula, const void* dy, const void* h, void* 
   void* a0[] = {&dy, &h, &dx, &dresidual, &part, &weight, &rstd, &M, &N};
   int rc = launch(name, dim3(parts), dim3(64 * waves), 0, stream, a0);
   if (rc) return rc;
-  snprintf(name, sizeof name, "teeny_rmsnorm_dw_reduce_%s", dtype_tag(dtype));
+  snprintf(name, sizeof name, "teeny_rmsnorm_dw_reduce_%s%s", few ? "few_" : "", dtype_tag(dtype));
   void* a1[] = {&part, &dweight, &parts, &N, &add_dw};
-  return launch(name, dim3((N + 31) / 32), dim3(1024), 0, stream, a1);
+  return few ? launch(name, dim3((N + 63) / 64), dim3(64), 0, stream, a1)
+             : launch(name, dim3((N + 31) / 32), dim3(1024), 0, stream, a1);
 }
 
 int teeny_fused_add_rmsnorm_bwd(const void* dy, const void* h, void* dx, void* dresidual,

@@ -177,7 +177,8 @@ struct Raw<bf16, 8> {
 
 // Wavefronts per workgroup: the registers of a row (dy, h, w, the dweight
 // sums) allow 4, 2 or 1 wavefronts per SIMD, all in one workgroup per CU, so
-// that the dweight partials stay one per workgroup.
+// that the dweight partials stay one per workgroup.  With few rows the host
+// launches the same kernels with 4 wavefronts.
 template <typename T, int VEC, int CH>
 constexpr int bwd_waves() {
   constexpr int B = CH * VEC * (int)sizeof(T);  // bytes of a row per lane
@@ -213,8 +214,9 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const
     for (int j = 0; j < VEC; ++j) dwacc[c][j] = 0.0f;
   }
   const float n_inv = 1.0f / (float)N;
-  const int stride = gridDim.x * NW;
-  int row = blockIdx.x * NW + wave;
+  const int waves = blockDim.x >> 6;  // NW, or fewer
+  const int stride = gridDim.x * waves;
+  int row = blockIdx.x * waves + wave;
   Raw<T, VEC> dyr[CH], hr[CH], dyn[PIPE ? CH : 1], hn[PIPE ? CH : 1];
   float rs = 0.0f, rsn = 0.0f;
   auto load = [&](int r, Raw<T, VEC>* a, Raw<T, VEC>* b, float& s) __attribute__((always_inline)) {
@@ -277,6 +279,7 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const
   }
 #pragma unroll
   for (int s = NW / 2; s >= 1; s /= 2) {
+    if (s >= waves) continue;
     if (wave >= s && wave < 2 * s)
 #pragma unroll
       for (int c = 0; c < CH; ++c)
@@ -332,6 +335,25 @@ __device__ void dw_reduce(const float* __restrict__ part, T* __restrict__ dw, in
   st(dw + n, (add ? ld(dw + n) : 0.0f) + s);
 }
 
+// The same for up to kFewParts partials (up to 64 rows), a thread per column
+// with every load in flight: the 1024 threads and the LDS sum cost a call of
+// one row 0.4 us.
+constexpr int kFewParts = 16;
+template <typename T>
+__device__ void dw_reduce_few(const float* __restrict__ part, T* __restrict__ dw, int nparts,
+                              int N, int add) {
+  const int n = blockIdx.x * 64 + threadIdx.x;
+  if (n >= N) return;
+  const float d0 = add ? ld(dw + n) : 0.0f;
+  float v[kFewParts], s = 0.0f;
+#pragma unroll
+  for (int p = 0; p < kFewParts; ++p) v[p] = part[(long)min(p, nparts - 1) * N + n];
+#pragma unroll
+  for (int p = 0; p < kFewParts; ++p)
+    if (p < nparts) s += v[p];
+  st(dw + n, d0 + s);
+}
+
 }  // namespace
 
 extern "C" __global__ __launch_bounds__(1024) void teeny_rmsnorm_dw_reduce_f32(
@@ -342,6 +364,16 @@ extern "C" __global__ __launch_bounds__(1024) void teeny_rmsnorm_dw_reduce_f32(
 extern "C" __global__ __launch_bounds__(1024) void teeny_rmsnorm_dw_reduce_bf16(
     const float* part, bf16* dw, int nparts, int N, int add) {
   dw_reduce(part, dw, nparts, N, add);
+}
+
+extern "C" __global__ __launch_bounds__(64) void teeny_rmsnorm_dw_reduce_few_f32(
+    const float* part, float* dw, int nparts, int N, int add) {
+  dw_reduce_few(part, dw, nparts, N, add);
+}
+
+extern "C" __global__ __launch_bounds__(64) void teeny_rmsnorm_dw_reduce_few_bf16(
+    const float* part, bf16* dw, int nparts, int N, int add) {
+  dw_reduce_few(part, dw, nparts, N, add);
 }
 
 // Few rows (a decode step's M = batch): one 256-thread workgroup per row, so

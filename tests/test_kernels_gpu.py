@@ -201,10 +201,10 @@ def test_rmsnorm_bf16_bwd(cuda, m, n):
 @pytest.mark.parametrize("m,n,dtype", [
     (m, n, t) for t in (torch.float32, torch.bfloat16)
     for m, n in [(1, 8), (15, 33), (17, 520), (4099, 512), (8200, 40), (33, 1032), (300, 2048),
-                 (70, 4096), (9, 3000), (21, 1023)]] + [(5, 8192, torch.bfloat16)])
+                 (70, 4096), (9, 3000), (21, 1023), (64, 520), (65, 520)]] + [(5, 8192, torch.bfloat16)])
 def test_rmsnorm_bwd_edges(cuda, m, n, dtype):
     """Backward at the edges of its workgroups (4, 8 or 16 rows), of the row
-    chunks and of the dweight reduction (32 columns, 1 to 256 partials), both
+    chunks and of the dweight reductions (1 to 16 and 1 to 256 partials), both
     formulas, against float64 on the stored inputs.  fp32: sums of n (dx) and m
     (dweight) terms, 2^-24 sqrt(terms) of the largest value; bf16: one rounding
     more (2^-8 of each value)."""
@@ -217,7 +217,12 @@ def test_rmsnorm_bwd_edges(cuda, m, n, dtype):
     want = {"ref": r * ww * (d - x * r * r * dot), "true": r * (ww * d - x * r * r * dot)}
     dw_want = (d * x * r).sum(0)
     dx_ref, dres, dw_ref = ops.fused_add_rmsnorm_bwd(dy, h, w, rstd)
+    ops._lib.profile_enable(True)
     dx_true, dw_true = ops.rmsnorm_bwd(dy, h, w, rstd)
+    names = ops._lib.profile_stats()
+    ops._lib.profile_enable(False)
+    # up to 64 rows: workgroups of 4 wavefronts, a thread per dweight column
+    assert any("dw_reduce_few" in x for x in names) == (m <= 64)
     assert torch.equal(dx_ref, dres) and torch.equal(dw_ref, dw_true)
     # a dweight written whole is the one accumulated into zeros
     zeros = lambda: torch.zeros_like(w)  # noqa: E731
