@@ -494,19 +494,25 @@ int teeny_qkv_rope_split_partials_dev(const float* parts, int n_parts, void* q_o
  * attends to cache rows 0 .. min(p + 1, cache_len) - 1 as by
  * teeny_decode_attention_dev; o [batch, Hq, D].  bf16, D 64 or 128,
  * Hq / Hkv <= 32; no workspace.  One workgroup per (b, kv head) reads that
- * head's rows, so it suits caches of a few thousand rows; longer ones
- * spread better over the split-K teeny_decode_attention_dev.  No reference
- * counterpart (the reference has no KV cache). */
+ * head's rows, so it suits steps over a thousand rows or many sequences;
+ * others share them as below.  No reference counterpart (the reference has no
+ * KV cache). */
 int teeny_decode_qkv_attention_dev(const float* parts, int n_parts, void* k_cache,
                                    void* v_cache, void* o, int batch, int n_heads_q,
                                    int n_heads_kv, int head_dim, int cache_len,
                                    const int32_t* n_past, float ln_rope_base,
                                    float softmax_scale, int dtype, hipStream_t stream);
 /* The same with each (b, kv head)'s keys shared by n_split workgroups, whose
- * partials (in the workspace) a second kernel merges: for long caches and few
- * sequences.  teeny_decode_qkv_attention_splits gives the measured choice, 1
- * where the one-launch form above is faster; the workspace is
- * teeny_decode_qkv_attention_workspace_bytes (0 for one split). */
+ * partials (in the workspace) a second kernel merges: for many keys and few
+ * sequences.  teeny_decode_qkv_attention_splits_at gives the measured choice
+ * for a step that attends n_keys rows of the cache (*n_past + 1; a captured
+ * step takes the most it will attend, or is captured for few and for many),
+ * 1 where the one-launch form above is faster;
+ * teeny_decode_qkv_attention_splits is that of a full cache of heads of 128.
+ * The workspace is teeny_decode_qkv_attention_workspace_bytes (0 for one
+ * split). */
+int teeny_decode_qkv_attention_splits_at(int batch, int n_heads_kv, int head_dim, int cache_len,
+                                         int n_keys);
 int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len);
 size_t teeny_decode_qkv_attention_workspace_bytes(int batch, int n_heads_q, int head_dim,
                                                   int n_split);

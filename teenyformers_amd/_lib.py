@@ -79,6 +79,7 @@ _SIGNATURES = {
                                    + [_f, _i, _p, _sz, _p], _i),
     "teeny_decode_qkv_attention_dev": ([_p, _i, _p, _p, _p] + [_i] * 5 + [_p, _f, _f, _i, _p],
                                        _i),
+    "teeny_decode_qkv_attention_splits_at": ([_i] * 5, _i),
     "teeny_decode_qkv_attention_splits": ([_i] * 3, _i),
     "teeny_decode_qkv_attention_workspace_bytes": ([_i] * 4, _sz),
     "teeny_decode_qkv_attention_split_dev": ([_p, _i, _p, _p, _p] + [_i] * 5 + [_p, _f, _f, _i, _i,

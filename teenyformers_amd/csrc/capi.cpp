@@ -1082,19 +1082,29 @@ int teeny_qkv_rope_split_partials_dev(const float* parts, int n_parts, void* q_o
 // Workgroups that share the keys of a (b, kv head) in the one-launch decode
 // attention: a key tile (32) per wavefront at full cache at the finest, until
 // every CU has a workgroup, at most 16 (32 was 0-50 % slower than 16).
-// Measured in a graph, 32 q and 8 kv heads of 128, us unsplit against this:
-// one sequence 1001 of 1100 keys 11.5 -> 10.5, 3901 of 4096 26.4 -> 11.7,
-// 12001 of 12200 111 -> 18.5 (30 through the unfused kernels); 8 sequences
-// 3901 of 4096 47.5 -> 31.9; an almost empty long cache (501 of 4096) 8.1 ->
-// 9.9, the merge's launch.  Up to 1024 rows and from half the CUs' worth of
-// (b, kv head) pairs it does not pay (16 sequences, 1001 of 1200: 18.2, 20.1
-// with 2; 640 rows, one sequence: 9.2, 9.8 with 4).
-int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len) {
-  if (batch <= 0 || n_heads_kv <= 0 || cache_len <= 0) return 0;
+// Measured in a graph, us unsplit and split; Hq32 Hkv8 D128 in a cache of 4096:
+//   keys          251         501         801         1031        2001        3901
+//   1 sequence    6.4,  9.4   7.7,  9.3   10.1, 9.3   11.9, 10.1  16.2, 10.5  25.9, 11.1
+//   8 sequences   7.4, 10.7   8.8, 11.5   11.2, 12.6  16.3, 14.7  29.2, 20.1  46.8, 31.1
+//   10 (3 shares)                         14.6, 15.3  17.7, 16.4  30.1, 22.6
+// and 12001 of 12200 keys of one sequence 111, 18.4.  So the keys attended
+// decide, not the cache: the merge's launch pays from about 1024.  With heads of
+// 64, half the bytes, 16 pairs of (b, kv head) cross there too (1031 keys 9.0,
+// 8.4), 64 pairs later (1031 9.3, 10.4; 1301 10.3, 10.7; 2001 14.3, 13.0).  Two
+// shares do not pay anywhere (Hq32 Hkv8 D128, 11 to 15 sequences, 1101 keys 18.6
+// to 20.1, 19.3 to 21.3; 24 x Hkv4 D64 2001 keys 16.9, 18.4; 16 to 31 sequences
+// of Hkv8, up to 3901 keys: 51.8 to 89.8, 54.6 to 95.5).
+int teeny_decode_qkv_attention_splits_at(int batch, int n_heads_kv, int head_dim, int cache_len,
+                                         int n_keys) {
+  if (batch <= 0 || n_heads_kv <= 0 || head_dim <= 0 || cache_len <= 0 || n_keys <= 0) return 0;
   const long wgs = (long)batch * n_heads_kv;
-  if (cache_len <= 1024 || 2 * wgs >= device_cus()) return 1;
-  const long s = std::min((long)device_cus() / wgs, (long)(cache_len + 255) / 256);
-  return s < 2 ? 1 : s > 16 ? 16 : (int)s;
+  const long s = std::min((long)device_cus() / wgs, std::min((long)(cache_len + 255) / 256, 16L));
+  const int least = head_dim >= 128 || wgs <= 32 ? 1024 : 2048;
+  return s < 3 || std::min(n_keys, cache_len) <= least ? 1 : (int)s;
+}
+
+int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len) {
+  return teeny_decode_qkv_attention_splits_at(batch, n_heads_kv, 128, cache_len, cache_len);
 }
 
 size_t teeny_decode_qkv_attention_workspace_bytes(int batch, int n_heads_q, int head_dim,

@@ -293,7 +293,8 @@ class Llama:
                 and cfg.head_dim() in (64, 128) and cfg.n_heads // cfg.n_kv_heads() <= 32
                 and cache.capacity * cfg.head_dim() * 2 < 2 ** 31
                 and (cache.capacity <= 4096
-                     or ops.decode_qkv_splits(qkv.shape[0], cfg.n_kv_heads(), cache.capacity) > 1))
+                     or ops.decode_qkv_splits(qkv.shape[0], cfg.n_kv_heads(), cache.capacity,
+                                              cfg.head_dim()) > 1))
 
     def _decode_ws(self, B: int, cache: KVCache, device) -> torch.Tensor:
         """Split-K workspace for decode attention over the whole cache."""

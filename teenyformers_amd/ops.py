@@ -546,19 +546,24 @@ def decode_attention(q, k_cache, v_cache, n_keys: int, softmax_scale: float | No
     return out
 
 
-def decode_qkv_splits(batch: int, n_heads_kv: int, cache_len: int) -> int:
-    """How many workgroups share each (b, kv head)'s keys in decode_qkv_attention."""
-    return _lib.lib().teeny_decode_qkv_attention_splits(batch, n_heads_kv, cache_len)
+def decode_qkv_splits(batch: int, n_heads_kv: int, cache_len: int, head_dim: int = 128,
+                      n_keys: int | None = None) -> int:
+    """How many workgroups share each (b, kv head)'s keys in a decode_qkv_attention
+    that attends n_keys rows of the cache (by default all of them)."""
+    return _lib.lib().teeny_decode_qkv_attention_splits_at(
+        batch, n_heads_kv, head_dim, cache_len, cache_len if n_keys is None else n_keys)
 
 
 def decode_qkv_attention(qkv: "Partials", k_cache, v_cache, n_past, n_heads_q: int,
                          n_heads_kv: int, rope_base: float, softmax_scale: float | None = None,
-                         out=None):
-    """A one-token step's attention in one launch (long caches of few
+                         out=None, n_keys: int | None = None):
+    """A one-token step's attention in one launch (many keys of few
     sequences: two, the second merging key splits): qkv (the QKV projection's
     K-split Partials, [B, 1, (Hq+2Hkv) D]) is split with RoPE at position
     *n_past (a one-element int32 device tensor), k / v are written to cache
-    row *n_past, and q attends to rows 0 .. *n_past.  Returns o [B, Hq, D]."""
+    row *n_past, and q attends to rows 0 .. *n_past.  Returns o [B, Hq, D].
+    n_keys: *n_past + 1 where the host knows it, by default the cache's
+    length; it only picks the number of key splits."""
     if not isinstance(qkv, Partials):
         raise TypeError("decode_qkv_attention takes the QKV projection's K-split slabs")
     _dev(qkv.slabs, k_cache, v_cache)
@@ -571,8 +576,8 @@ def decode_qkv_attention(qkv: "Partials", k_cache, v_cache, n_past, n_heads_q: i
     scale = 1.0 / math.sqrt(D) if softmax_scale is None else float(softmax_scale)
     out = torch.empty((B, n_heads_q, D), dtype=k_cache.dtype, device=k_cache.device) \
         if out is None else out
-    # few sequences over a long cache share each kv head's keys between workgroups
-    splits = decode_qkv_splits(B, n_heads_kv, L)
+    # few sequences of many keys share each kv head's keys between workgroups
+    splits = decode_qkv_splits(B, n_heads_kv, L, D, n_keys)
     need = _lib.lib().teeny_decode_qkv_attention_workspace_bytes(B, n_heads_q, D, splits)
     ws = torch.empty(need, dtype=torch.uint8, device=out.device) if need else None
     call("teeny_decode_qkv_attention_split_dev", _p(qkv.slabs), qkv.n, _p(k_cache), _p(v_cache),
