@@ -220,9 +220,11 @@ class Llama:
         return self.sw.get(name, self.w[name])
 
     # -- one block (src/layers/llama_block.rs:55-65) -------------------------
-    def _attention(self, i: int, n1: torch.Tensor, cache: KVCache, pos0) -> torch.Tensor:
+    def _attention(self, i: int, n1: torch.Tensor, cache: KVCache, pos0,
+                   n_keys: int | None = None) -> torch.Tensor:
         """src/layers/attention.rs:83-148 with GQA and a KV cache.  pos0: an int,
-        or (one-token decode in a captured graph) an int32 device tensor."""
+        or (one-token decode in a captured graph) an int32 device tensor; n_keys:
+        as in hidden."""
         cfg, w = self.cfg, self.w
         B, S, d = n1.shape
         Hq, Hkv, D = cfg.n_heads, cfg.n_kv_heads(), cfg.head_dim()
@@ -234,7 +236,7 @@ class Llama:
         if isinstance(pos0, torch.Tensor) and self._fused_decode(qkv, cache):
             # one launch: QKV split, RoPE, cache write and attention
             o = ops.decode_qkv_attention(qkv, cache.k[i], cache.v[i], pos0, Hq, Hkv,
-                                         cfg.rope_base, scale)
+                                         cfg.rope_base, scale, n_keys=n_keys)
             return ops.linear_split(o.view(B, 1, Hq * D), self._lw(p + "o_proj.weight"), rows=rows)
         if (not isinstance(pos0, torch.Tensor) and pos0 == 0
                 and not isinstance(qkv, ops.Partials) and qkv.dtype == torch.bfloat16):
@@ -310,15 +312,19 @@ class Llama:
         f = ops.linear_swiglu(n2, self._lw(p + "gate_up_proj.weight"))
         return ops.linear_split(f, self._lw(p + "down_proj.weight"), rows=ops.split_rows())
 
-    def hidden(self, ids: torch.Tensor, cache: KVCache, pos0, trace: list | None = None
-               ) -> torch.Tensor:
+    def hidden(self, ids: torch.Tensor, cache: KVCache, pos0, trace: list | None = None,
+               n_keys: int | None = None) -> torch.Tensor:
         """Final-norm hidden states [B, S, d] for ids [B, S] at positions pos0..,
         appending the new keys/values to `cache` (pos0 may be an int32 device
         tensor for one-token steps; cache.length is then left to the caller).
         trace: if a list, each block appends (x, attn, x + attn, ffn): its
         input residual stream, the attention sub-layer's output, the stream
         after the attention add, and the FFN output (the block's output is
-        the sum of the last two)."""
+        the sum of the last two).  n_keys: with a device position, the cache
+        rows that the step attends (the position plus one) where the host knows
+        them, as it does of an int; by default the whole cache.  Only the
+        number of workgroups that share them depends on it (a captured step
+        with decode_step's bits gives n_keys of its replays' range)."""
         cfg, w = self.cfg, self.w
         eps = cfg.eps
         x, n1 = ops.embed_rmsnorm(ids, w["model.embed_tokens.weight"],
@@ -328,13 +334,14 @@ class Llama:
             # a one-token step takes its position from device memory, as the
             # captured graph does, so both run the same kernels
             pos = torch.tensor([pos0], dtype=torch.int32, device=ids.device)
+            n_keys = pos0 + 1
         delta = None
         for i in range(cfg.n_layers):
             p = f"model.layers.{i}."
             if i > 0:  # x = x + ffn(...) fused into this block's input norm
                 n1, x, _ = ops.fused_add_rmsnorm(delta, x, w[p + "input_layernorm.weight"], eps)
             x_in = x
-            a = self._attention(i, n1, cache, pos)
+            a = self._attention(i, n1, cache, pos, n_keys)
             n2, x, _ = ops.fused_add_rmsnorm(a, x, w[p + "post_attention_layernorm.weight"], eps)
             delta = self._ffn(i, n2)
             if trace is not None:
@@ -344,9 +351,9 @@ class Llama:
             cache.length = pos0 + ids.shape[1]
         return y
 
-    def logits(self, h: torch.Tensor) -> torch.Tensor:
-        """Tied lm_head (src/layers/embedding.rs:159-167): h @ E^T."""
-        return ops.linear(h, self._lw("model.embed_tokens.weight"))
+    def logits(self, h: torch.Tensor, out: torch.Tensor | None = None) -> torch.Tensor:
+        """Tied lm_head (src/layers/embedding.rs:159-167): h @ E^T (into out, if given)."""
+        return ops.linear(h, self._lw("model.embed_tokens.weight"), out)
 
     def forward(self, ids: torch.Tensor) -> torch.Tensor:
         """All-position logits [B, S, vocab] (src/llama.rs:65-81)."""
@@ -449,7 +456,12 @@ class DecodeGraph:
     replayed step's logits.  trace: a list that the captured step's blocks
     append their sub-layer tensors to (as Llama.hidden's trace); after each
     replay they hold that step's values.  Positions past the cache capacity
-    are not written (the kernels check)."""
+    are not written (the kernels check).
+    A cache in which steps over few and over many keys both lie ahead has two
+    captures of the step, which differ in the workgroups that share a kv
+    head's keys (ops.decode_qkv_splits); replay() takes the one that an eager
+    step of its length would run.  With a trace there is one, of the first
+    captured length."""
 
     def __init__(self, model: Llama, cache: KVCache, ids: torch.Tensor,
                  trace: list | None = None):
@@ -460,29 +472,48 @@ class DecodeGraph:
         side = torch.cuda.Stream()
         side.wait_stream(torch.cuda.current_stream())
         with torch.cuda.stream(side):
-            self._step()
+            self.first_logits = self._step(cache.length + 1)
         torch.cuda.current_stream().wait_stream(side)
         torch.cuda.synchronize()
-        self.first_logits = self.logits
         cache.length += 1
-        self.graph = torch.cuda.CUDAGraph()
-        with torch.cuda.graph(self.graph):
-            self._step(trace)
+        self.logits = torch.empty_like(self.first_logits)
+        self.graph = None
+        self._graphs = {}  # by the number of key splits
+        for n_keys in (cache.length + 1, cache.capacity) if trace is None else (cache.length + 1,):
+            splits = self._splits(n_keys)
+            if splits not in self._graphs:
+                g = torch.cuda.CUDAGraph()
+                # one pool: the captures are never replayed at the same time
+                with torch.cuda.graph(g, pool=self.graph.pool() if self.graph else None):
+                    self._step(n_keys, trace, self.logits)
+                self._graphs[splits] = g
+                self.graph = self.graph or g
 
-    def _step(self, trace: list | None = None):
+    def _splits(self, n_keys: int) -> int:
+        """The key splits of a step that attends n_keys rows (1 where the step
+        does not run the fused attention)."""
+        cfg, cache = self.model.cfg, self.cache
+        if cache.k[0].dtype != torch.bfloat16 or cfg.head_dim() not in (64, 128):
+            return 1
+        return ops.decode_qkv_splits(self.ids.shape[0], cfg.n_kv_heads(), cache.capacity,
+                                     cfg.head_dim(), n_keys)
+
+    def _step(self, n_keys: int, trace: list | None = None, logits: torch.Tensor | None = None
+              ) -> torch.Tensor:
         m = self.model
         # the eager first step runs the kernels the capture records (the
         # library's own at any batch, as teeny_linear_bf16 under capture)
         with ops.own_gemm():
-            h = m.hidden(self.ids, self.cache, self.pos, trace=trace)
-            self.logits = m.logits(h[:, -1])
+            h = m.hidden(self.ids, self.cache, self.pos, trace=trace, n_keys=n_keys)
+            logits = m.logits(h[:, -1], logits)
             # the greedy choice lands in the ids the next replay embeds (the
             # embedding read them at the start of this step)
             # (and the position moves on: every kernel that reads it came before)
-            ops.argmax_rows(self.logits, out=self.ids.view(-1), advance=self.pos)
+            ops.argmax_rows(logits, out=self.ids.view(-1), advance=self.pos)
+        return logits
 
     def replay(self):
         if self.cache.length >= self.cache.capacity:
             raise RuntimeError("KV cache is full")
-        self.graph.replay()
+        self._graphs.get(self._splits(self.cache.length + 1), self.graph).replay()
         self.cache.length += 1

@@ -688,39 +688,48 @@ class StreamWeight:
         return self.w.shape
 
 
+def _product_out(x2: torch.Tensor, n: int, out: torch.Tensor | None) -> torch.Tensor:
+    return torch.empty((x2.shape[0], n), dtype=x2.dtype, device=x2.device) if out is None else out
+
+
 def _row_major(w):
     return w.w if isinstance(w, StreamWeight) else w
 
 
-def linear(x: torch.Tensor, w) -> torch.Tensor:
+def linear(x: torch.Tensor, w, out: torch.Tensor | None = None) -> torch.Tensor:
     """y = x w^T (src/layers/mod.rs:54-58; w [out, in]) through the library:
     bf16 by teeny_linear_bf16 (up to 16 rows stream the weight through the
     decode kernels, more rows run hipBLASLt, or this library's GEMM under
     own_gemm()), fp32 (the reference's precision) by teeny_linear_f32.
     Products that need a gradient use torch's GEMM (the library's linear
-    kernels have no backward).  w may be a StreamWeight."""
+    kernels have no backward).  w may be a StreamWeight.  out: where y goes, a
+    contiguous tensor of its shape, type and device."""
     x2 = x.reshape(-1, x.shape[-1])
     N, K = w.shape
     if K != x2.shape[1]:
         raise ValueError(f"linear: x has {x2.shape[1]} features, w expects {K}")
+    if out is not None and (out.shape != (*x.shape[:-1], N) or out.dtype != x.dtype
+                            or out.device != x.device or not out.is_contiguous()):
+        raise ValueError("linear: out must be contiguous, of y's shape, type and device")
     if isinstance(w, StreamWeight):
         if _skinny(x2, w.w, N):
             x2 = x2.contiguous()
-            y = torch.empty((x2.shape[0], N), dtype=x.dtype, device=x.device)
+            y = _product_out(x2, N, out)
             call("teeny_linear_rows_bf16", _p(x2), _p(w.s), _p(y), x2.shape[0], N, K,
                  _lib.TEENY_LINEAR_PLAIN, K, 1, _stream())
             return y.view(*x.shape[:-1], N)
         w = w.w
     if _gemm_f32(x2, w):
         x2 = x2.contiguous()
-        y = torch.empty((x2.shape[0], N), dtype=x.dtype, device=x.device)
+        y = _product_out(x2, N, out)
         fn = "teeny_gemm_f32" if getattr(_own_gemm, "on", False) else "teeny_linear_f32"
         call(fn, _p(x2), _p(w), _p(y), x2.shape[0], N, K, _stream())
         return y.view(*x.shape[:-1], N)
     if not _gemm(x2, w):
-        return torch.nn.functional.linear(x, w)
+        y = torch.nn.functional.linear(x, w)
+        return y if out is None else out.copy_(y)
     x2 = x2.contiguous()
-    y = torch.empty((x2.shape[0], N), dtype=x.dtype, device=x.device)
+    y = _product_out(x2, N, out)
     fn = ("teeny_gemm_bf16" if x2.shape[0] > 16 and getattr(_own_gemm, "on", False)
           else "teeny_linear_bf16")
     call(fn, _p(x2), _p(w), _p(y), x2.shape[0], N, K, _stream())

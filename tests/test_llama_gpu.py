@@ -423,6 +423,37 @@ def test_captured_hidden_equals_decode_step(cuda, batch):
         assert torch.equal(got, want)
 
 
+def test_decode_graph_across_key_splits(cuda):
+    """A cache whose steps pass from unsplit attention to key splits (more than
+    1024 keys): each replay has the bits of the eager step of its length, in
+    the one logits tensor, and the steps over few keys run the unsplit kernel
+    whatever the capacity."""
+    cfg = llama.LlamaConfig(d_model=512, n_heads=8, n_layers=2, vocab_size=512, eps=1e-5,
+                            rope_base=1e4, intermediate_size=1024, n_kv_heads_=2)
+    model = llama.Llama(cfg, llama.init_weights(cfg, dtype=torch.bfloat16, std=0.2, seed=33))
+    g = torch.Generator(device="cuda").manual_seed(34)
+    prompt = torch.randint(0, 512, (2, 1019), generator=g, device="cuda")
+    cache, logits = model.prefill(prompt, 1032)
+    eager, _ = model.prefill(prompt, 1032)
+    ids = ops.argmax_rows(logits).view(-1, 1)
+    dg = llama.DecodeGraph(model, cache, ids)
+    assert sorted(dg._graphs) == [1, 5]
+    assert torch.equal(dg.first_logits, model.decode_step(eager, ids))
+    held = dg.logits
+    for _ in range(11):  # 1021 .. 1031 keys
+        ids = dg.ids.clone()
+        names = []
+        ops._lib.profile_enable(True)
+        want = model.decode_step(eager, ids)
+        names = ops._lib.profile_stats()
+        ops._lib.profile_enable(False)
+        dg.replay()
+        torch.cuda.synchronize()
+        assert dg.logits is held and torch.equal(held, want), eager.length
+        assert ("teeny_decode_qkv_attn_split_bf16_d64" in names) == (eager.length > 1024)
+        assert ("teeny_decode_qkv_attn_bf16_d64" in names) == (eager.length <= 1024)
+
+
 def test_generate_stream_layout_equals_row_major(cuda):
     """Greedy ids of the graph-replayed decode with the weights in the
     streaming layout (ops.StreamWeight) == the eager decode from the
