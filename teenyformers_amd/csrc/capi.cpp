@@ -1091,16 +1091,18 @@ int teeny_qkv_rope_split_partials_dev(const float* parts, int n_parts, void* q_o
 // decide, not the cache: the merge's launch pays from about 1024.  With heads of
 // 64, half the bytes, 16 pairs of (b, kv head) cross there too (1031 keys 9.0,
 // 8.4), 64 pairs later (1031 9.3, 10.4; 1301 10.3, 10.7; 2001 14.3, 13.0).  Two
-// shares do not pay anywhere (Hq32 Hkv8 D128, 11 to 15 sequences, 1101 keys 18.6
-// to 20.1, 19.3 to 21.3; 24 x Hkv4 D64 2001 keys 16.9, 18.4; 16 to 31 sequences
-// of Hkv8, up to 3901 keys: 51.8 to 89.8, 54.6 to 95.5).
+// shares pay from twice the keys: Hkv8 D128, 11 and 15 sequences, 1101 keys
+// 18.6, 19.3 and 20.1, 21.3; 2501 33.0, 28.0 and 35.9, 34.3; 4001 49.6, 39.6 and
+// 52.8, 51.7; Hkv4 D64, 22 and 31 sequences, 2001 17.0, 17.7 and 18.4, 19.6;
+// 4001 27.6, 25.9 and 31.1, 30.4.  From 128 pairs on they do not (16 sequences
+// of Hkv8 D128, 2001 to 4001 keys 32.1 to 53.3, 32.0 to 55.4; 24, 78.9, 88.8).
 int teeny_decode_qkv_attention_splits_at(int batch, int n_heads_kv, int head_dim, int cache_len,
                                          int n_keys) {
   if (batch <= 0 || n_heads_kv <= 0 || head_dim <= 0 || cache_len <= 0 || n_keys <= 0) return 0;
   const long wgs = (long)batch * n_heads_kv;
   const long s = std::min((long)device_cus() / wgs, std::min((long)(cache_len + 255) / 256, 16L));
-  const int least = head_dim >= 128 || wgs <= 32 ? 1024 : 2048;
-  return s < 3 || std::min(n_keys, cache_len) <= least ? 1 : (int)s;
+  const int least = (s == 2 ? 2048 : 1024) * (head_dim >= 128 || wgs <= 32 ? 1 : 2);
+  return s < 2 || 2 * wgs >= device_cus() || std::min(n_keys, cache_len) <= least ? 1 : (int)s;
 }
 
 int teeny_decode_qkv_attention_splits(int batch, int n_heads_kv, int cache_len) {

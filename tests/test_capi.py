@@ -276,18 +276,20 @@ def test_fa2_32bit_row_offsets(L):
 
 def test_decode_qkv_attention_splits(L):
     """Key splits of the fused decode attention on a 256-CU device (here,
-    without a GPU to ask): at least three workgroups per (b, kv head), at most
-    16, and only for the keys attended that pay the merge."""
+    without a GPU to ask): at most 16 workgroups per (b, kv head), and only
+    for the keys attended that pay the merge."""
     at = L.teeny_decode_qkv_attention_splits_at
     assert [at(1, 8, 128, 4096, n) for n in (1, 1024, 1025, 4096, 9999)] == [1, 1, 16, 16, 16]
-    assert [at(b, 8, 128, 4096, 4096) for b in (2, 4, 8, 10, 11, 16, 64)] == [16, 8, 4, 3, 1, 1, 1]
+    assert [at(b, 8, 128, 4096, 4096) for b in (2, 4, 8, 10, 11, 16, 64)] == [16, 8, 4, 3, 2, 1, 1]
+    assert [at(15, 8, 128, 4096, n) for n in (2048, 2049)] == [1, 2]  # two shares: twice the keys
     assert at(1, 8, 128, 1100, 1100) == 5  # a key tile per wavefront
     # heads of 64: half the bytes, from 33 (b, kv head) pairs on twice the keys
     assert [at(16, 2, 64, 4096, n) for n in (1024, 1025)] == [1, 8]
     assert [at(33, 1, 64, 4096, n) for n in (2048, 2049)] == [1, 7]
+    assert [at(31, 4, 64, 8192, n) for n in (4096, 4097)] == [1, 2]
     assert at(0, 8, 128, 4096, 1) == at(1, 8, 128, 4096, 0) == 0
     assert [L.teeny_decode_qkv_attention_splits(1, 8, n) for n in (1024, 4096)] == [1, 16]
-    assert L.teeny_decode_qkv_attention_splits(24, 4, 4096) == 1
+    assert L.teeny_decode_qkv_attention_splits(11, 8, 1100) == 1
 
 
 def test_decode_qkv_attention_32bit_cache_offsets(L):
