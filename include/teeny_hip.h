@@ -416,10 +416,10 @@ int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F
 /* The same Linear in fp32, the reference's precision (teeny-core's Linear
  * behind sym_linear, src/layers/mod.rs:54-58, on the f32 weights that
  * src/loader.rs:41,66-80 decodes): hipBLASLt's fp32 GEMM (fp32 products
- * and accumulation, no workspace), or teeny_gemm_f32 for up to 4 rows and
- * where hipBLASLt does not take the device or shape or the stream is
- * capturing.  Any M and N; K
- * a multiple of 4; x and w 16-byte aligned. */
+ * and accumulation, no workspace), or teeny_gemm_f32 for up to 4 rows with K
+ * up to 2048 (5120 from N 65536) and where hipBLASLt does not take the device
+ * or shape or the stream is capturing.  Any M and N; K a multiple of 4; x and
+ * w 16-byte aligned. */
 int teeny_linear_f32(const void* x, const void* w, void* y, int M, int N, int K,
                      hipStream_t stream);
 /* This library's fp32 GEMM for the same product: each output fp32 fused

@@ -1401,17 +1401,23 @@ int teeny_gemm_f32(const void* x, const void* w, void* y, int M, int N, int K,
                 args);
 }
 
-// hipBLASLt's fp32 GEMM (no workspace), or teeny_gemm_f32 for up to 4 rows and
-// where hipBLASLt does not take the device or shape, or the stream is
-// capturing.
+// hipBLASLt's fp32 GEMM (no workspace), or teeny_gemm_f32 for up to 4 rows of
+// short products and where hipBLASLt does not take the device or shape, or the
+// stream is capturing.
 int teeny_linear_f32(const void* x, const void* w, void* y, int M, int N, int K,
                      hipStream_t stream) {
   int rc = gemm_f32_check(x, w, y, M, N, K);
   if (rc) return rc;
-  // up to 4 rows the own kernel reads w faster (M 1, N 32000 K 2048: 44 us
-  // against 60; N 3072 K 2048: 8 against 14; M 4, N 28672 K 4096: 87 against
-  // 100, N 4096 K 14336: 42.6 against 43.7), from 8 rows the library at large K
-  if (M <= 4) return teeny_gemm_f32(x, w, y, M, N, K, stream);
+  // up to 4 rows the own kernel reads w faster up to K 2048 and for the largest
+  // N; a workgroup walks the whole K, so with few workgroups or a long K the
+  // library is ahead.  Own and library, us, M 1 / M 4 (14 N of 128 to 128256 at
+  // 13 K of 256 to 14336): K 256 N 4096 3.2 / 3.2 and 10.2 / 9.9; K 2048 N 3072
+  // 7.3 / 7.7 and 10.2; N 32768 44 / 47 and 59; K 4096 N 128256 349 / 356 and
+  // 453 / 456; but K 4096 N 4096 16.6 / 17.2 and 15.4, K 8192 N 6144 51 / 54 and
+  // 39, K 14336 N 512 33 / 37 and 25; from K 2560 it depends on N either way.  The
+  // one loss inside the rule: K 1536 N 49152 46 / 54 and 46.
+  if (M <= 4 && (K <= 2048 || (N >= 65536 && K <= 5120)))
+    return teeny_gemm_f32(x, w, y, M, N, K, stream);
   if (teeny_lt_gemm_f32(x, w, y, M, N, K, stream) == 0) return TEENY_OK;
   return teeny_gemm_f32(x, w, y, M, N, K, stream);
 }

@@ -209,6 +209,21 @@ def test_gemm_f32_few_rows(cuda, M, N, K):
     assert torch.equal(y, _gemm_f32(xd, wd, "teeny_gemm_f32")[:M])
 
 
+@pytest.mark.parametrize("M,N,K,own", [
+    (1, 256, 2048, True), (4, 256, 2048, True), (5, 256, 512, False), (4, 256, 2052, False),
+    (4, 65536, 2052, True), (1, 65532, 2052, False), (1, 256, 14336, False)])
+def test_linear_f32_route(cuda, M, N, K, own):
+    """Up to 4 rows run the own kernel where it is the faster one: short K, or
+    the largest N."""
+    x, w = torch.randn(M, K, device="cuda"), torch.randn(N, K, device="cuda")
+    ops._lib.profile_enable(True)
+    y = ops.linear(x, w)
+    names = ops._lib.profile_stats()
+    ops._lib.profile_enable(False)
+    assert any("gemm_f32_sk" in n for n in names) == own
+    assert torch.allclose(y.double(), x.double() @ w.double().t(), rtol=0, atol=K * 2.0 ** -20)
+
+
 def test_linear_f32_op(cuda):
     """ops.linear routes fp32 products (no gradient) through teeny_linear_f32,
     not torch; ops.gemm_f32 is the own kernel."""
