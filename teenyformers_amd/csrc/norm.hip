@@ -215,6 +215,7 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const
   }
   const float n_inv = 1.0f / (float)N;
   const int waves = blockDim.x >> 6;  // NW, or fewer
+  const int active = min(waves, M - (int)blockIdx.x * waves);  // that have a row
   const int stride = gridDim.x * waves;
   int row = blockIdx.x * waves + wave;
   Raw<T, VEC> dyr[CH], hr[CH], dyn[PIPE ? CH : 1], hn[PIPE ? CH : 1];
@@ -279,7 +280,7 @@ __device__ __forceinline__ void rmsnorm_bwd_rows(const T* __restrict__ dy, const
   }
 #pragma unroll
   for (int s = NW / 2; s >= 1; s /= 2) {
-    if (s >= waves) continue;
+    if (s >= active) continue;
     if (wave >= s && wave < 2 * s)
 #pragma unroll
       for (int c = 0; c < CH; ++c)
@@ -345,12 +346,20 @@ __device__ void dw_reduce_few(const float* __restrict__ part, T* __restrict__ dw
   const int n = blockIdx.x * 64 + threadIdx.x;
   if (n >= N) return;
   const float d0 = add ? ld(dw + n) : 0.0f;
-  float v[kFewParts], s = 0.0f;
+  float s = 0.0f;
+  auto sum = [&](auto count) {
+    constexpr int C = decltype(count)::value;
+    float v[C];
 #pragma unroll
-  for (int p = 0; p < kFewParts; ++p) v[p] = part[(long)min(p, nparts - 1) * N + n];
+    for (int p = 0; p < C; ++p) v[p] = part[(long)min(p, nparts - 1) * N + n];
 #pragma unroll
-  for (int p = 0; p < kFewParts; ++p)
-    if (p < nparts) s += v[p];
+    for (int p = 0; p < C; ++p)
+      if (p < nparts) s += v[p];
+  };
+  if (nparts <= 4)
+    sum(std::integral_constant<int, 4>{});
+  else
+    sum(std::integral_constant<int, kFewParts>{});
   st(dw + n, d0 + s);
 }
 
