@@ -448,12 +448,22 @@ int fa2_bwd(bool causal, const void* q, const void* k, const void* v, const void
     long total = (long)nmb * batch * (pack ? hkv : hq);
     if (total >= (1L << 31)) return TEENY_ERR_INVALID_SHAPE;
     int tot = (int)total;
-    // at most one workgroup a CU and a long walk: two wavefront groups share
-    // its keys (backward, 1 group against 2: B1 Hq8 Hkv2 S4096 D128 185 and
-    // 170 us, B1 Hq8 Hkv1 S3125 D128 140 and 131, B1 H16 S2048 D64 79 and 74,
-    // B1 Hq32 Hkv8 S1021 D64 53 and 51; shorter walks pay more for the second
-    // group's Q, dO and O rows: S1024 D128 equal, S300 D64 20.0 and 20.6)
-    const bool k2 = total <= device_cus() && n_ctx_k >= 15 * head_dim;
+    // at most one workgroup a CU and a long walk over the keys that it sees:
+    // two wavefront groups share them, which pays from some 10 head sizes of
+    // keys; the line has a margin.  Backward, us, 1 group and 2:
+    //   keys                   300         512         768         960
+    //   B1 H16 D64 causal      19.5, 20.2  26.8, 26.8  36.4, 35.1  42.0, 40.4
+    //   B1 Hq32 Hkv8 D64 c.    27.5, 28.3  33.4, 33.5  42.9, 41.6  48.8, 46.8
+    //   B2 H8 Sq256 D64        17.5, 18.2  19.7, 19.8  23.5, 22.3  26.4, 24.9
+    //   keys                   512         1024        1500-1536   1920
+    //   B1 H16 D128 causal     37.4, 38.4  59.3, 58.6  84.8, 82.0  102.3, 98.9
+    //   B1 Hq8 Hkv1 D128 c.    42.0, 43.3  62.1, 60.7  78.1, 75.5  89.6, 85.3
+    //   B2 H8 Sq256 D128       27.6, 29.1  37.9, 37.5  48.6, 45.9  56.9, 52.5
+    // and H16 S2048 78.8, 74.1 (D64) and 108.1, 104.6 (D128), Hq8 Hkv1 S3125 D128
+    // 134.5, 125.7.  Causal rows see no key past the last query: B2 H16 Sq536
+    // Sk2500 D128 with fp32 gradients 57.1, 61.5.
+    const int walk = causal ? std::min(n_ctx_q, n_ctx_k) : n_ctx_k;
+    const bool k2 = total <= device_cus() && walk >= 15 * head_dim;
     snprintf(name, sizeof name, "teeny_fa2_bwd_dq_bf16_d%d_%s%s%s%s", head_dim, cz,
              pack ? "_g4" : "", k2 ? "_k2" : "", gsfx);
     void* a2[] = {&q,       &k,       &v,     &o,  &dout, &l,   &ld,  &dq,

@@ -18,7 +18,7 @@ import pytest
 import torch
 
 from oracle import oracle as O
-from teenyformers_amd import ops
+from teenyformers_amd import _lib, ops
 
 pytestmark = pytest.mark.gpu
 
@@ -78,6 +78,16 @@ def check_flat(name, got, want):
     r = rel_l2(got, want)
     assert err <= BF16_MAX_ABS and (r is None or r <= BF16_REL_L2), \
         f"{name}: max abs {err:.3e}, rel-L2 {r}"
+
+
+def launched(f):
+    """f's result and the names of the library's kernels that it launched."""
+    _lib.profile_enable(True)
+    try:
+        out = f()
+        return out, sorted(_lib.profile_stats())
+    finally:
+        _lib.profile_enable(False)
 
 
 def inputs(seed, B, Hq, Hkv, Sq, Sk, D, bf16, spike=False):
@@ -540,23 +550,34 @@ def test_fa2_bf16_bwd_shared_walk(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32)
     (1, 4, 1, 1025, 1025, 64, True),   # GQA groups of 4: blocks of one tile (none for group 1) to 17
     (1, 1, 1, 33, 960, 64, False),     # 15 tiles, the shortest walk taken
     (2, 2, 1, 1, 1023, 64, False),     # one row, a last tile of 63 keys
-    (1, 4, 1, 64, 1985, 128, True),    # one tile a block, keys past every row
+    (1, 4, 1, 64, 1985, 128, True),    # keys past every row: a short walk after all
+    (1, 2, 2, 970, 1100, 64, True),    # keys past every row beside a long walk
     (1, 1, 1, 1930, 1930, 128, True),
     (1, 2, 2, 130, 1921, 128, False),  # 31 tiles, the last of one key
 ])
 def test_fa2_bf16_bwd_dq_two_key_groups(cuda, B, Hq, Hkv, Sq, Sk, D, causal, grad_f32):
     """dQ whose keys two wavefront groups of a workgroup share (few rows, long
-    walks), against the oracle at the bf16 bar, twice with the same bits."""
+    walks), against the oracle, twice with the same bits.  bf16 gradients at
+    the bf16 bar; fp32 ones at the flat bar, and dQ's error, 2^-17 of dS's
+    operand rounding (hi + lo) against the stored bf16's 2^-9, at most a
+    sixteenth of the bf16 gradient's."""
     q, k, v, do = inputs(67, B, Hq, Hkv, Sq, Sk, D, bf16=True)
     scale = 1.0 / math.sqrt(D)
     qd, kd, vd, dod = (dev(t, torch.bfloat16) for t in (q, k, v, do))
     o, lse = ops.flash_attn2_fwd(qd, kd, vd, scale, causal)
-    a = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
-    b = ops.flash_attn2_bwd(qd, kd, vd, o, lse, dod, scale, causal, grad_f32=grad_f32)
+    run = lambda g32: ops.flash_attn2_bwd(  # noqa: E731
+        qd, kd, vd, o, lse, dod, scale, causal, grad_f32=g32)
+    a, names = launched(lambda: run(grad_f32))
+    dq_names = [n for n in names if "_bwd_dq_" in n]
+    walk = min(Sq, Sk) if causal else Sk
+    assert len(dq_names) == 1 and ("_k2" in dq_names[0]) == (walk >= 15 * D), names
+    b = run(grad_f32)
     assert all(torch.equal(x, y) for x, y in zip(a, b))
     want = O.fa2_bwd(q, k, v, host(o), do, host(lse), scale, causal)
     for name, got, w in zip(("dq", "dk", "dv"), a, want):
-        check_bf16(name, host(got), w)
+        (check_flat if grad_f32 else check_bf16)(name, host(got), w)
+    if grad_f32:
+        assert rel_l2(host(a[0]), want[0]) <= rel_l2(host(run(False)[0]), want[0]) / 16
 
 
 def _random_shapes(n, seed=2026):
