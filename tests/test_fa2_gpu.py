@@ -185,9 +185,13 @@ def test_fa2_f32_edges(cuda, shape, causal, aligned):
     oe, le = O.fa2_fwd(q, k, v, scale, causal)
     assert np.abs(host(o) - oe).max() <= F32_TOL
     assert np.abs(host(lse) - le).max() <= F32_TOL
-    grads = ops.flash_attn2_bwd(qd, kd, vd, put(oe), lse, dod, scale, causal,
-                                dq=put(np.zeros_like(q)), dk=put(np.zeros_like(k)),
-                                dv=put(np.zeros_like(v)))
+    grads, names = launched(lambda: ops.flash_attn2_bwd(
+        qd, kd, vd, put(oe), lse, dod, scale, causal, dq=put(np.zeros_like(q)),
+        dk=put(np.zeros_like(k)), dv=put(np.zeros_like(v))))
+    # walks of at least two shares of four q tiles are shared out (their merge
+    # stores whole vectors)
+    shared = Hq // Hkv * math.ceil(Sq / 32) >= 8
+    assert ("teeny_fa2_dkdv_merge_bf16_g32" in names) == (shared and aligned)
     for name, got, want in zip(("dq", "dk", "dv"), grads, O.fa2_bwd(q, k, v, oe, do, le, scale, causal)):
         err = float(np.abs(host(got) - want).max())
         assert err <= F32_TOL * max(1.0, float(np.abs(want).max())), f"{name} {err}"

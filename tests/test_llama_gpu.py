@@ -346,6 +346,7 @@ def test_decode_qkv_attention_fused(cuda, B, Hq, Hkv, D, L):
     wq = _bf16_dev((0.05 * rng.standard_normal((n, d))).astype(np.float32))
     pq = ops.linear_split(x, wq, 128)
     assert pq.n == 4
+    assert (ops.decode_qkv_splits(B, Hkv, L) > 1) == (L > 1024)
     kc0 = _bf16_dev(rng.standard_normal((B, Hkv, L, D)).astype(np.float32))
     vc0 = _bf16_dev(rng.standard_normal((B, Hkv, L, D)).astype(np.float32))
     scale = 1.0 / math.sqrt(D)
