@@ -398,16 +398,18 @@ int teeny_argmax_rows_advance(const void* x, int64_t* out, int rows, int cols, i
  * first, src/loader.rs:49-55); writes y[M, F] = silu(x w_gate^T) *
  * (x w_up^T) with both products rounded to bf16 first, as FeedForward's
  * gate_up Linear followed by SwigluOp computes it (src/layers/ffn.rs:47-56),
- * without writing the [M, 2F] product: up to 16 rows with F % 64 == 0 and
+ * without writing the [M, 2F] product: up to 64 rows with F % 64 == 0 and
  * K % 128 == 0 take the weight-streaming kernel, other shapes the GEMM with
  * the SwiGLU in its epilogue (F % 32 == 0 and K % 64 == 0, otherwise
- * TEENY_ERR_UNSUPPORTED).  Bit-identical to teeny_linear_bf16 on [2F, K]
+ * TEENY_ERR_UNSUPPORTED).  Bit-identical to teeny_gemm_bf16 on [2F, K]
  * followed by teeny_swiglu_fwd. */
 int teeny_linear_bf16(const void* x, const void* w, void* y, int M, int N, int K,
                       hipStream_t stream);
-/* This library's matrix-core GEMM for the same product, any M (N and K
- * multiples of 64): teeny_linear_bf16's fallback above 16 rows, and the
- * kernel whose epilogue forms teeny_linear_swiglu_bf16 at those sizes. */
+/* This library's own kernels for the same product, any M (N and K multiples
+ * of 64, K below 2^22): teeny_linear_bf16's fallback above 16 rows.  Up to 64
+ * rows with N % 128 == 0 and K % 128 == 0 they stream the weight, as the decode
+ * kernels do; otherwise the matrix-core GEMM whose epilogue forms
+ * teeny_linear_swiglu_bf16. */
 int teeny_gemm_bf16(const void* x, const void* w, void* y, int M, int N, int K,
                     hipStream_t stream);
 int teeny_linear_swiglu_bf16(const void* x, const void* w, void* y, int M, int F, int K,

@@ -352,11 +352,12 @@ int device_cus() {
 //     partial sums a merge kernel adds in a fixed order (needs the larger
 //     workspace).
 // Measured (MI355X, causal, Hq/Hkv 4 and 8, D 64 and 128, same-box A/B of
-// every combination): two groups are 1.02-1.45x the plain kernel from 2048
-// to 8191 query rows and at least as fast as any split there; from 12288
-// rows of one sequence the 4-way split is 1.05-1.13x and the two groups
-// 0.98-1.05x; at 512 and 1024 rows, for the bidirectional kernel and with
-// many key-block workgroups (B2 S8192) the plain kernel is fastest.
+// every combination of these forms): two groups are 1.02-1.45x the plain kernel
+// from 2048 to 8191 query rows; from 12288 rows of one sequence the 4-way split
+// is 1.05-1.13x and the two groups 0.98-1.05x; at 512 and 1024 rows, for the
+// bidirectional kernel and with many key-block workgroups (B2 S8192) the plain
+// kernel is fastest.  dkdv_share, below, replaces the plain kernel and the two
+// groups where the key blocks leave CUs idle.
 struct DkdvPlan {
   int groups, split;
 };

@@ -1,8 +1,9 @@
 // bf16 GEMM on the gfx950 matrix cores: y[M, N] = x[M, K] . w[N, K]^T with
 // fp32 accumulation, y rounded to bf16 (nearest even).  This is the Linear
 // behind sym_linear (reference src/layers/mod.rs:54-58: external teeny-core
-// Linear, W [out, in], no bias) at prompt sizes; decode-step sizes (M <= 16)
-// run the weight-streaming kernels of linear_bf16.hip instead.
+// Linear, W [out, in], no bias) at prompt sizes; decode-step sizes (M <= 64
+// with N and K multiples of 128) run the weight-streaming kernels of
+// linear_bf16.hip instead.
 //
 // Both operands are K-contiguous rows, which is exactly the operand form of
 // v_mfma_f32_32x32x16_bf16 (each lane holds 8 consecutive k of one row), so

@@ -3,7 +3,8 @@
 // runs in fp32; src/loader.rs:41,66-80 decodes every weight to f32).
 //
 // teeny_linear_f32 hands its products to hipBLASLt; these kernels are the
-// library's own path where hipBLASLt does not take the device, shape or
+// library's own path for up to 4 rows of short products (the rule and its
+// figures: capi.cpp) and where hipBLASLt does not take the device, shape or
 // stream (a product under graph capture).
 //
 // Up to 64 rows (a decode step, one row per sequence): teeny_gemm_f32_sk_*,

@@ -699,7 +699,7 @@ def _row_major(w):
 def linear(x: torch.Tensor, w, out: torch.Tensor | None = None) -> torch.Tensor:
     """y = x w^T (src/layers/mod.rs:54-58; w [out, in]) through the library:
     bf16 by teeny_linear_bf16 (up to 16 rows stream the weight through the
-    decode kernels, more rows run hipBLASLt, or this library's GEMM under
+    decode kernels, more rows run hipBLASLt, or this library's kernels under
     own_gemm()), fp32 (the reference's precision) by teeny_linear_f32.
     Products that need a gradient use torch's GEMM (the library's linear
     kernels have no backward).  w may be a StreamWeight.  out: where y goes, a
@@ -761,13 +761,13 @@ def gemm_own(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 def linear_swiglu(x: torch.Tensor, w_gate_up) -> torch.Tensor:
-    """swiglu(x w_gate_up^T) (src/layers/ffn.rs:47-56).  Up to 16 bf16 rows
-    without gradients: one launch of teeny_linear_swiglu_bf16 (the decode
-    kernel with the SwiGLU fused).  More rows: the linear entry point
-    (hipBLASLt) and then the SwiGLU kernel, measured faster than the own GEMM
-    with the SwiGLU epilogue (1.40 against 1.52 ms at 8192 x 28672 x 4096);
-    other cases: the GEMM followed by the SwiGLU kernel.  w_gate_up may be a
-    StreamWeight."""
+    """swiglu(x w_gate_up^T) (src/layers/ffn.rs:47-56).  Up to split_rows() bf16
+    rows (16, or 64 in a decode step) without gradients: one launch of
+    teeny_linear_rows_bf16 (the decode kernel with the SwiGLU fused).  More
+    rows: the linear entry point (hipBLASLt) and then the SwiGLU kernel,
+    measured faster than the own GEMM with the SwiGLU epilogue (1.40 against
+    1.52 ms at 8192 x 28672 x 4096); other cases: the GEMM followed by the
+    SwiGLU kernel.  w_gate_up may be a StreamWeight."""
     x2 = x.reshape(-1, x.shape[-1])
     N2, K = w_gate_up.shape
     if K != x2.shape[1] or N2 % 2:
